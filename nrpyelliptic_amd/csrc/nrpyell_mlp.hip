@@ -19,7 +19,9 @@
 #include "nrpyell_internal.h"
 
 typedef __bf16 bf16_t;
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 #define MLP_K0 64  // input features, zero-padded so every GEMM dimension is a multiple of 64
@@ -32,7 +34,17 @@ struct MlpOffsets {
   long w[MLP_HIDDEN + 2], b[MLP_HIDDEN + 2];
 };
 
-__device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + __expf(-z)); }
+// 1 / (1 + e^-z). The reciprocal is v_rcp_f32 (1 ulp) with one Newton step, and v_div_fixup_f32
+// restores the quotient's special values (1 / inf = 0, NaN): 4 instructions in the place of the
+// 10 of an FP32 division. Measured over 4 million z in [-30, 30], z * sigmoidf_(z) is the same
+// float as with the division (largest relative error against FP64 1.8e-6, from the exponential;
+// below z = -87.3, where the sigmoid is a denormal, it is 0).
+__device__ __forceinline__ float sigmoidf_(float z) {
+  const float d = 1.0f + __expf(-z);
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  return __builtin_amdgcn_div_fixupf(r, d, 1.0f);
+}
 __device__ __forceinline__ bf16_t to_bf16(float x) { return (bf16_t)x; }
 
 // splitmix64 of (seed, m): the dataset row of minibatch row m (uniform, with replacement)
@@ -80,8 +92,8 @@ __device__ __forceinline__ long swz(int row, int col, int inner16) {
   return ((long)((row >> 5) * inner16 + (col >> 4)) * 64 + ((col >> 3) & 1) * 32 + (row & 31)) * 8 + (col & 7);
 }
 
-// Where the BF16 weight copies live: pw[k] = bf16(p[k]) (row-major, for inference) and, in
-// pws, W_l (rows n, inner k; l = 1..5) and W_l^T (rows k, inner n; l = 2..5) in the operand layout.
+// Where the BF16 weight copies live in pws: W_l (rows n, inner k; l = 1..5) and W_l^T (rows k,
+// inner n; l = 2..5) in the operand layout.
 struct WeightCopies {
   long w_off[MLP_HIDDEN + 1];  // W_l in the FP32 parameters
   long fs[MLP_HIDDEN + 1];     // W_l in pws
@@ -413,95 +425,134 @@ __global__ void __launch_bounds__(256) mlp_wgrad_kernel(WgradArgs a) {
   }
 }
 
-// Inference, all six layers in one launch: a block takes 64 rows through the five hidden
-// layers with the activations held in LDS (two 64 x 256 BF16 buffers, ping-pong), so nothing
-// but the 64 input features and the output leave the chip; the pre-activations are not kept
-// (training uses the per-layer kernels, whose backward needs them). Each of the 4 waves owns 64
-// output columns: 2 x 2 MFMA accumulators over the 64 rows; the weights (544 KB of BF16, shared
-// by every block) are read from L2 as 16-byte MFMA operands. Same arithmetic as the per-layer
-// path: FP32 accumulation over BF16 operands in ascending K, z = acc + b, h = bf16(silu(z)),
+// Inference, all six layers in one launch: a block takes FI_R rows through the five hidden
+// layers with the activations held in LDS (one FI_R x 256 BF16 buffer, overwritten layer by
+// layer), so nothing but the 64 input features and the output leave the chip. Arithmetic of an
+// entry: FP32 accumulation over BF16 products in ascending K, z = acc + b, h = bf16(silu(z)),
 // output y = sum_k h_k w_k + b in FP32.
+//
+// Each of the 4 waves owns 64 output columns of the 64 rows, as 2 x 2 MFMA accumulators of
+// Z^T = W H^T: with the weights as the first operand a lane ends up with 4 consecutive columns of
+// one row, i.e. one 8-byte LDS store instead of four 2-byte ones, and the weights (544 KB of
+// BF16, shared by every block) come from the operand layout, 1 KB of consecutive bytes per wave
+// and load, FI_PF inner steps ahead of their use and across the layer boundary. The kernel is
+// bound by the activations' vector instructions (1280 per row, each an exponential, a reciprocal
+// and about 8 more; the MFMAs need 58 us of the 186 at 2.5 PFLOP/s) and overlaps them with other
+// waves' MFMAs: four blocks per CU, which the single buffer (40 KB of LDS) and 124 registers per
+// lane allow. 262 144 rows: 186 us, 786 TFLOP/s (two ping-pong buffers, row-major weights loaded
+// where they are used and FP32 divisions: 390 us, 375 TFLOP/s; the same outputs).
 constexpr int FI_R = 64, FI_LD = MLP_W + 8;  // rows per block; LDS row stride (528 B)
+constexpr int FI_PF = 4;                     // inner steps of weights in flight
 
-__global__ void __launch_bounds__(256) mlp_forward_fused_kernel(const bf16_t *__restrict__ X, const bf16_t *__restrict__ pw,
-                                                                const float *__restrict__ p, MlpOffsets off, int M,
-                                                                float *__restrict__ y) {
-  __shared__ __attribute__((aligned(16))) bf16_t Hbuf[2][FI_R * FI_LD];
+// One hidden layer of K inputs: acc[x][y] (columns 64 wave + 32 x .., rows 32 y ..) from the
+// activations in H, with the first FI_PF weight steps of this wave's two column tiles already in wv.
+template <int K>
+__device__ __forceinline__ void fi_layer(const bf16_t *H, const bf16_t *__restrict__ W, bf16x8 (&wv)[FI_PF][2],
+                                         floatx16 (&acc)[2][2]) {
+  constexpr int Q = K / 16;
+#pragma unroll
+  for (int x = 0; x < 2; x++)
+#pragma unroll
+    for (int y = 0; y < 2; y++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[x][y][r] = 0.0f;
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    bf16x8 h[2];
+#pragma unroll
+    for (int y = 0; y < 2; y++) h[y] = *(const bf16x8 *)(H + 32 * y * FI_LD + 16 * q);
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int y = 0; y < 2; y++)
+        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[q % FI_PF][x], h[y], acc[x][y], 0, 0, 0);
+    if (q + FI_PF < Q) {
+#pragma unroll
+      for (int x = 0; x < 2; x++) wv[q % FI_PF][x] = *(const bf16x8 *)(W + ((long)x * Q + q + FI_PF) * 512);
+    }
+  }
+}
+
+__global__ void __launch_bounds__(256, 3) mlp_forward_fused_kernel(const bf16_t *__restrict__ X,
+                                                                   const bf16_t *__restrict__ pws,
+                                                                   const float *__restrict__ p, MlpOffsets off,
+                                                                   WeightCopies wc, int M, float *__restrict__ y) {
+  __shared__ __attribute__((aligned(16))) bf16_t Hbuf[FI_R * FI_LD];
+  __shared__ __attribute__((aligned(16))) float s_b[MLP_HIDDEN][MLP_W];
   __shared__ float s_out[4][FI_R];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 31, lj = lane >> 5;
   const int r0 = blockIdx.x * FI_R;
+  bf16x8 wv[FI_PF][2];
+  const bf16_t *W = pws + wc.fs[1] + (long)(2 * wave) * (MLP_K0 / 16) * 512 + 8 * lane;
+#pragma unroll
+  for (int q = 0; q < FI_PF; q++)
+#pragma unroll
+    for (int x = 0; x < 2; x++) wv[q][x] = *(const bf16x8 *)(W + (x * (MLP_K0 / 16) + q) * 512);
   // input features: 64 rows x 64 BF16 = 512 chunks of 16 B, 2 per thread (rows past M clamped)
 #pragma unroll
   for (int q = 0; q < 2; q++) {
     const int e = tid + 256 * q, row = e >> 3, ch = e & 7;
     const int m = min(r0 + row, M - 1);
-    *(bf16x8 *)(&Hbuf[0][row * FI_LD + 8 * ch]) = *(const bf16x8 *)(X + (long)m * MLP_K0 + 8 * ch);
+    *(bf16x8 *)(&Hbuf[row * FI_LD + 8 * ch]) = *(const bf16x8 *)(X + (long)m * MLP_K0 + 8 * ch);
   }
+#pragma unroll
+  for (int l = 0; l < MLP_HIDDEN; l++) s_b[l][tid] = p[off.b[l + 1] + tid];
   __syncthreads();
-  int cur = 0;
-  const int wc = wave * 64;
+  const bf16_t *H = Hbuf + li * FI_LD + 8 * lj;
   for (int l = 1; l <= MLP_HIDDEN; l++) {
-    const int Kl = l == 1 ? MLP_K0 : MLP_W;
-    const bf16_t *W = pw + off.w[l];  // W_l [256 x K_l]
     floatx16 acc[2][2];
+    if (l == 1)
+      fi_layer<MLP_K0>(H, W, wv, acc);
+    else
+      fi_layer<MLP_W>(H, W, wv, acc);
+    if (l < MLP_HIDDEN) {  // the next layer's first weights, in flight during the activations
+      W = pws + wc.fs[l + 1] + (long)(2 * wave) * (MLP_W / 16) * 512 + 8 * lane;
 #pragma unroll
-    for (int x = 0; x < 2; x++)
+      for (int q = 0; q < FI_PF; q++)
 #pragma unroll
-      for (int yy = 0; yy < 2; yy++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[x][yy][r] = 0.0f;
-    const bf16_t *Hin = Hbuf[cur];
-    for (int k = 0; k < Kl; k += 16) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int x = 0; x < 2; x++) a[x] = *(const bf16x8 *)(Hin + (32 * x + li) * FI_LD + k + 8 * lj);
-#pragma unroll
-      for (int yy = 0; yy < 2; yy++) b[yy] = *(const bf16x8 *)(W + (long)(wc + 32 * yy + li) * Kl + k + 8 * lj);
-#pragma unroll
-      for (int x = 0; x < 2; x++)
-#pragma unroll
-        for (int yy = 0; yy < 2; yy++)
-          acc[x][yy] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x], b[yy], acc[x][yy], 0, 0, 0);
+        for (int x = 0; x < 2; x++) wv[q][x] = *(const bf16x8 *)(W + (x * (MLP_W / 16) + q) * 512);
     }
-    bf16_t *Hout = Hbuf[cur ^ 1];
-    const float *bias = p + off.b[l];
-    // accumulator r of lane (li, lj) in tile (x, yy): row 8*(r/4) + 4*lj + r%4, column li
+    __syncthreads();  // every wave has read this layer's input
+    // accumulator r of lane (li, lj) in tile (x, yy): column 8*(r/4) + 4*lj + r%4, row li
 #pragma unroll
     for (int x = 0; x < 2; x++)
 #pragma unroll
-      for (int yy = 0; yy < 2; yy++) {
-        const int c = wc + 32 * yy + li;
-        const float bc = bias[c];
+      for (int g = 0; g < 4; g++) {
+        const int c = 64 * wave + 32 * x + 8 * g + 4 * lj;
+        const float4 b = *(const float4 *)(&s_b[l - 1][c]);
+        const float bb[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int row = 32 * x + 8 * (r >> 2) + 4 * lj + (r & 3);
-          const float z = acc[x][yy][r] + bc;
-          Hout[row * FI_LD + c] = to_bf16(z * sigmoidf_(z));
+        for (int yy = 0; yy < 2; yy++) {
+          floatx4 h;
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const float z = acc[x][yy][4 * g + i] + bb[i];
+            h[i] = z * sigmoidf_(z);
+          }
+          *(bf16x4 *)(&Hbuf[(32 * yy + li) * FI_LD + c]) = __builtin_convertvector(h, bf16x4);
         }
       }
     __syncthreads();
-    cur ^= 1;
   }
   // output layer: wave w sums columns 64w..64w+63 of every row, then the 4 partials are added
-  const bf16_t *Hl = Hbuf[cur];
-  const float *wout = p + off.w[MLP_HIDDEN + 1];
-  for (int row = lane; row < FI_R; row += 64) {
-    float acc = 0.0f;
-#pragma unroll 8
-    for (int c = 0; c < 64; c++) acc += (float)Hl[row * FI_LD + wc + c] * wout[wc + c];
-    s_out[wave][row] = acc;
+  const float *wout = p + off.w[MLP_HIDDEN + 1] + 64 * wave;
+  float acc = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 64; c += 8) {
+    const bf16x8 h = *(const bf16x8 *)(&Hbuf[lane * FI_LD + 64 * wave + c]);
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc += (float)h[i] * wout[c + i];
   }
+  s_out[wave][lane] = acc;
   __syncthreads();
   if (tid < FI_R && r0 + tid < M)
     y[r0 + tid] = ((s_out[0][tid] + s_out[1][tid]) + (s_out[2][tid] + s_out[3][tid])) + p[off.b[MLP_HIDDEN + 1]];
 }
 
 // the BF16 copies of parameter k (see WeightCopies)
-__device__ __forceinline__ void store_weight(const WeightCopies &wc, long k, float v, bf16_t *__restrict__ pw,
-                                             bf16_t *__restrict__ pws) {
+__device__ __forceinline__ void store_weight(const WeightCopies &wc, long k, float v, bf16_t *__restrict__ pws) {
   const bf16_t b = to_bf16(v);
-  pw[k] = b;
 #pragma unroll
   for (int l = 1; l <= MLP_HIDDEN; l++) {
     const int Kl = l == 1 ? MLP_K0 : MLP_W;
@@ -514,10 +565,10 @@ __device__ __forceinline__ void store_weight(const WeightCopies &wc, long k, flo
   }
 }
 
-__global__ void refresh_weights_kernel(long n, const float *__restrict__ p, WeightCopies wc, bf16_t *__restrict__ pw,
+__global__ void refresh_weights_kernel(long n, const float *__restrict__ p, WeightCopies wc,
                                        bf16_t *__restrict__ pws) {
   const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) store_weight(wc, k, p[k], pw, pws);
+  if (k < n) store_weight(wc, k, p[k], pws);
 }
 
 // g = sum of the TR_SPLITS partials in range order; with update, an Adam step on p and the
@@ -525,7 +576,7 @@ __global__ void refresh_weights_kernel(long n, const float *__restrict__ p, Weig
 __global__ void mlp_adam_kernel(long n, const float *__restrict__ part, float *__restrict__ g, int update,
                                 float *__restrict__ p, float *__restrict__ mo, float *__restrict__ ve, float lr,
                                 float b1, float b2, float eps, float c1, float c2, WeightCopies wc,
-                                bf16_t *__restrict__ pw, bf16_t *__restrict__ pws) {
+                                bf16_t *__restrict__ pws) {
   const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   float gk = 0.0f;
@@ -539,7 +590,7 @@ __global__ void mlp_adam_kernel(long n, const float *__restrict__ part, float *_
   ve[k] = v;
   const float pk = p[k] - lr * (m / c1) / (sqrtf(v / c2) + eps);
   p[k] = pk;
-  store_weight(wc, k, pk, pw, pws);
+  store_weight(wc, k, pk, pws);
 }
 
 __global__ void gather_rows_kernel(const bf16_t *__restrict__ X, const float *__restrict__ t, long N, int M,
@@ -690,7 +741,6 @@ struct nrpyell_mlp {
   long n_params = 0;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
   float *part = nullptr;  // per-range gradient partials [TR_SPLITS x n_params]
-  bf16_t *pw = nullptr;   // BF16 copy of all parameters (weights read by the MFMA kernels)
   bf16_t *pws = nullptr;  // BF16 W_l and W_l^T in the MFMA operand layout (WeightCopies)
   long adam_t = 0;
   int cap = 0;                       // minibatch arrays allocated for this many rows
@@ -708,7 +758,7 @@ struct nrpyell_mlp {
   hipStream_t st = nullptr;
   ~nrpyell_mlp() {
     (void)hipFree(p); (void)hipFree(g); (void)hipFree(m); (void)hipFree(v); (void)hipFree(part);
-    (void)hipFree(pw); (void)hipFree(pws); (void)hipFree(loss);
+    (void)hipFree(pws); (void)hipFree(loss);
     release_seed();
     release();
     if (st) (void)hipStreamDestroy(st);
@@ -774,7 +824,7 @@ struct nrpyell_mlp {
   static long pws_size() { return (long)MLP_W * MLP_K0 + (2L * MLP_HIDDEN - 2) * MLP_W * MLP_W; }
   void refresh_bf16() {
     hipLaunchKernelGGL(refresh_weights_kernel, dim3((n_params + 255) / 256), dim3(256), 0, st, n_params, p, copies(),
-                       pw, pws);
+                       pws);
   }
   // forward, loss (added to *loss_out) and gradient partials of M minibatch rows (M a multiple
   // of 64): rows drawn from the dataset (gather) or its first M rows
@@ -822,7 +872,7 @@ struct nrpyell_mlp {
       c2 = 1.0f - powf(b2, (float)adam_t);
     }
     hipLaunchKernelGGL(mlp_adam_kernel, dim3((n_params + 255) / 256), dim3(256), 0, st, n_params, part, g, update, p,
-                       m, v, lr, b1, b2, 1e-8f, c1, c2, copies(), pw, pws);
+                       m, v, lr, b1, b2, 1e-8f, c1, c2, copies(), pws);
   }
 };
 
@@ -866,7 +916,6 @@ extern "C" int nrpyell_mlp_create(unsigned long long seed, nrpyell_mlp **out) {
     s->g = mlp_alloc<float>(off);
     s->m = mlp_alloc<float>(off);
     s->v = mlp_alloc<float>(off);
-    s->pw = mlp_alloc<bf16_t>(off);
     s->pws = mlp_alloc<bf16_t>((size_t)nrpyell_mlp::pws_size());
     s->part = mlp_alloc<float>((size_t)TR_SPLITS * off);
     s->loss = mlp_alloc<double>(1);
@@ -922,13 +971,8 @@ static int check_rows(int M) {
 extern "C" int nrpyell_mlp_forward(nrpyell_mlp *s, const void *x, int M, float *y_out) {
   return api_call([&]() -> int {
     if (check_rows(M)) return NRPYELL_EINVAL;
-    MlpOffsets off;
-    for (int l = 1; l <= MLP_HIDDEN + 1; l++) {
-      off.w[l] = s->w_off[l];
-      off.b[l] = s->b_off[l];
-    }
     hipLaunchKernelGGL(mlp_forward_fused_kernel, dim3((M + FI_R - 1) / FI_R), dim3(256), 0, s->st, (const bf16_t *)x,
-                       s->pw, s->p, off, M, y_out);
+                       s->pws, s->p, s->offsets(), s->copies(), M, y_out);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->st));
     return NRPYELL_OK;
