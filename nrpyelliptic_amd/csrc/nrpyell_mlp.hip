@@ -476,13 +476,13 @@ __device__ __forceinline__ void fi_layer(const bf16_t *H, const bf16_t *__restri
 __global__ void __launch_bounds__(256, 3) mlp_forward_fused_kernel(const bf16_t *__restrict__ X,
                                                                    const bf16_t *__restrict__ pws,
                                                                    const float *__restrict__ p, MlpOffsets off,
-                                                                   WeightCopies wc, int M, float *__restrict__ y) {
+                                                                   WeightCopies wc, long M, float *__restrict__ y) {
   __shared__ __attribute__((aligned(16))) bf16_t Hbuf[FI_R * FI_LD];
   __shared__ __attribute__((aligned(16))) float s_b[MLP_HIDDEN][MLP_W];
   __shared__ float s_out[4][FI_R];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 31, lj = lane >> 5;
-  const int r0 = blockIdx.x * FI_R;
+  const long r0 = (long)blockIdx.x * FI_R;
   bf16x8 wv[FI_PF][2];
   const bf16_t *W = pws + wc.fs[1] + (long)(2 * wave) * (MLP_K0 / 16) * 512 + 8 * lane;
 #pragma unroll
@@ -493,8 +493,8 @@ __global__ void __launch_bounds__(256, 3) mlp_forward_fused_kernel(const bf16_t 
 #pragma unroll
   for (int q = 0; q < 2; q++) {
     const int e = tid + 256 * q, row = e >> 3, ch = e & 7;
-    const int m = min(r0 + row, M - 1);
-    *(bf16x8 *)(&Hbuf[row * FI_LD + 8 * ch]) = *(const bf16x8 *)(X + (long)m * MLP_K0 + 8 * ch);
+    const long m = min(r0 + row, M - 1);
+    *(bf16x8 *)(&Hbuf[row * FI_LD + 8 * ch]) = *(const bf16x8 *)(X + m * MLP_K0 + 8 * ch);
   }
 #pragma unroll
   for (int l = 0; l < MLP_HIDDEN; l++) s_b[l][tid] = p[off.b[l + 1] + tid];
@@ -620,8 +620,8 @@ struct FeatureParams {
   double m[2], pos[2][3], P[2][3], S[2][3];
 };
 
-__device__ inline void point_features(const FeatureParams &f, double x0, double x1, double x2, float out[MLP_K0],
-                                      double &scale) {
+__device__ inline void point_features(const FeatureParams &f, double x0, double x1, double x2,
+                                      float out[MLP_NFEAT], double &scale) {
   const double f0 = f.AMAX * (exp(x0 / f.w) - exp(-x0 / f.w)) / f.D;
   const double X = f0 * sin(x1) * cos(x2), Y = f0 * sin(x1) * sin(x2), Z = sqrt(f0 * f0 + f.b * f.b) * cos(x1);
   const double r = sqrt(X * X + Y * Y + Z * Z), rb = r + f.b;
@@ -649,30 +649,49 @@ __device__ inline void point_features(const FeatureParams &f, double x0, double 
   for (int n = 0; n < 2; n++)
     for (int d = 0; d < 3; d++) out[k++] = (float)(f.S[n][d] / fmax(f.m[n] * f.m[n], 1e-12));
   out[k++] = (float)(f.b / 10.0);
-  while (k < MLP_K0) out[k++] = 0.0f;
   scale = 1.0 / (50.0 * rb);
 }
 
-// One thread per interior or pure-outer point (i0 in [NG, G0), i1, i2 interior).
-__global__ void features_kernel(GridDims g, FeatureParams f, const double *xx0, const double *xx1, const double *xx2,
-                                bf16_t *__restrict__ X, double *__restrict__ scale, long *__restrict__ idx) {
-  const int n0 = g.G0 - NRPYELL_NG;
-  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// One thread per interior or pure-outer point (i0 in [NG, G0), i1, i2 interior) and per padding
+// row (zeros). The block's 256 rows of 128 B leave through LDS, so that a wave's store is 1 KB of
+// consecutive bytes: 272 384 rows in 18.7 us, now bound by the FP64 closed forms (64 two-byte stores per thread, 128 B apart, after
+// a clearing pass over X: 26 us and 10 us).
+constexpr int FEAT_C = (MLP_NFEAT + 7) / 8;  // 16-byte chunks of a row that hold features
+__global__ void __launch_bounds__(256) features_kernel(GridDims g, FeatureParams f, const double *__restrict__ xx0,
+                                                       const double *__restrict__ xx1, const double *__restrict__ xx2,
+                                                       long rows, bf16_t *__restrict__ X, double *__restrict__ scale,
+                                                       long *__restrict__ idx) {
+  __shared__ __attribute__((aligned(16))) bf16_t s_x[256][8 * FEAT_C];
+  const int n0 = g.G0 - NRPYELL_NG, tid = threadIdx.x;
+  const long k0 = (long)blockIdx.x * 256, k = k0 + tid;
   const long npts = (long)n0 * g.N1 * g.N2;
-  if (k >= npts) return;
-  const int i0 = NRPYELL_NG + (int)(k % n0);
-  const int i1 = NRPYELL_NG + (int)((k / n0) % g.N1);
-  const int i2 = NRPYELL_NG + (int)(k / ((long)n0 * g.N1));
-  float out[MLP_K0];
-  double s;
-  point_features(f, xx0[i0], xx1[i1], xx2[i2], out, s);
+  float out[MLP_NFEAT] = {};
+  if (k < npts) {
+    const int i0 = NRPYELL_NG + (int)(k % n0);
+    const int i1 = NRPYELL_NG + (int)((k / n0) % g.N1);
+    const int i2 = NRPYELL_NG + (int)(k / ((long)n0 * g.N1));
+    double s;
+    point_features(f, xx0[i0], xx1[i1], xx2[i2], out, s);
+    scale[k] = s;
+    idx[k] = idx3(g, i0, i1, i2);
+  }
 #pragma unroll
-  for (int q = 0; q < MLP_K0; q++) X[k * MLP_K0 + q] = to_bf16(out[q]);
-  scale[k] = s;
-  idx[k] = idx3(g, i0, i1, i2);
+  for (int q = 0; q < 8 * FEAT_C; q++) s_x[tid][q] = to_bf16(q < MLP_NFEAT ? out[q] : 0.0f);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < MLP_K0 / 8; q++) {
+    const int e = tid + 256 * q, row = e / (MLP_K0 / 8), ch = e % (MLP_K0 / 8);
+    bf16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = to_bf16(0.0f);
+    if (ch < FEAT_C) v = *(const bf16x8 *)(&s_x[row][8 * ch]);
+    if (k0 + row < rows) *(bf16x8 *)(X + (k0 + row) * MLP_K0 + 8 * ch) = v;
+  }
 }
 
-// u = t * scale at the listed points, v = eta u, and the parity images of each point.
+// u = e^t * scale at the listed points. FINAL: also v = eta u, and both at every parity image;
+// otherwise u and its images in the interior phi planes, which is what the smoothing reads.
+template <bool FINAL>
 __global__ void seed_state_kernel(GridDims g, long npts, const float *__restrict__ t, const double *__restrict__ scale,
                                   const long *__restrict__ idx, double eta, double *__restrict__ yn) {
   const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -680,41 +699,58 @@ __global__ void seed_state_kernel(GridDims g, long npts, const float *__restrict
   const double u = exp((double)t[k]) * scale[k];
   const long p = idx[k];
   yn[p] = u;
-  yn[g.ntot + p] = eta * u;
+  if (FINAL) yn[g.ntot + p] = eta * u;
   const int i0 = (int)(p % g.G0), i1 = (int)((p / g.G0) % g.G1), i2 = (int)(p / ((long)g.G0 * g.G1));
-  for_each_image(g, i0, i1, i2, [&](long d) {
-    yn[d] = u;
-    yn[g.ntot + d] = eta * u;
-  });
+  if (FINAL)
+    for_each_image(g, i0, i1, i2, [&](long d) {
+      yn[d] = u;
+      yn[g.ntot + d] = eta * u;
+    });
+  else
+    for_each_image_in_planes(g, i0, i1, i2, [&](long d) { yn[d] = u; });
 }
 
-// One binomial smoothing sub-pass of u along direction DIR over the interior points,
-// out = (u[-1] + 2 u + u[+1]) / 4 (phi neighbours through the periodic map), pure outer points
-// copied; every point writes its interior-plane parity images, so the next sub-pass reads
-// current ghosts. It removes the grid-scale part of the network's pointwise error (BF16
-// activations round independently at neighbouring points), which the Laplacian in the
-// residual would otherwise amplify by 1/dx^2.
-template <int DIR>
-__global__ void smooth_kernel(GridDims g, const double *__restrict__ in, double *__restrict__ out) {
+// One binomial smoothing pass of u over the interior points, (f[-1] + 2 f + f[+1]) / 4 along i0,
+// then i1, then i2 (phi neighbours through the periodic map), pure outer points copied. It removes
+// the grid-scale part of the network's pointwise error (BF16 activations round independently at
+// neighbouring points), which the Laplacian in the residual would otherwise amplify by 1/dx^2.
+// Every thread forms the i0 averages of its 3 x 3 (i1, i2) neighbours itself: on a ghost row they
+// are those of the row's source point, because `in` holds the parity images there and the average
+// is symmetric. So the three directions are one pass over memory (5.8 us at 128x128x16, LAST 8.5;
+// as three 5.1 + 5.3 + 6.2 us and a copy back, then 7 us for v and the ghost planes). Every point writes its images: those in the
+// interior phi planes for the next pass, LAST all of them and v = eta u beside u.
+template <bool LAST>
+__global__ void smooth_kernel(GridDims g, double eta, const double *__restrict__ in, double *__restrict__ out) {
   const int i0 = NRPYELL_NG + blockIdx.x * blockDim.x + threadIdx.x;
   const int i1 = NRPYELL_NG + blockIdx.y, i2 = NRPYELL_NG + blockIdx.z;
   if (i0 >= g.G0) return;
   const long p = idx3(g, i0, i1, i2);
   double v = in[p];
   if (i0 < g.N0 + NRPYELL_NG) {
-    long pm, pp;
-    if (DIR == 0) { pm = p - 1; pp = p + 1; }
-    else if (DIR == 1) { pm = p - g.G0; pp = p + g.G0; }
-    else { pm = idx3(g, i0, i1, wrap2(g, i2 - 1)); pp = idx3(g, i0, i1, wrap2(g, i2 + 1)); }
-    v = 0.25 * (in[pm] + in[pp]) + 0.5 * v;
+    double f2[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const int j2 = wrap2(g, i2 + k - 1);
+      double f1[3];
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        const double *f = in + idx3(g, i0, i1 + j - 1, j2);
+        f1[j] = 0.25 * (f[-1] + f[1]) + 0.5 * f[0];
+      }
+      f2[k] = 0.25 * (f1[0] + f1[2]) + 0.5 * f1[1];
+    }
+    v = 0.25 * (f2[0] + f2[2]) + 0.5 * f2[1];
   }
   out[p] = v;
-  for_each_image_in_planes(g, i0, i1, i2, [&](long d) { out[d] = v; });
-}
-
-__global__ void v_from_u_kernel(long n, double eta, double *y) {
-  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) y[n + k] = eta * y[k];
+  if (LAST) {
+    out[g.ntot + p] = eta * v;
+    for_each_image(g, i0, i1, i2, [&](long d) {
+      out[d] = v;
+      out[g.ntot + d] = eta * v;
+    });
+  } else {
+    for_each_image_in_planes(g, i0, i1, i2, [&](long d) { out[d] = v; });
+  }
 }
 
 // log(u / scale) at the listed points: the network's training target from a solved state
@@ -755,6 +791,8 @@ struct nrpyell_mlp {
   double *seed_scale = nullptr;
   long *seed_idx = nullptr;
   float *seed_y = nullptr;
+  int seed_nxx = 0;           // coordinates seed_xx has room for
+  double *seed_xx = nullptr;
   hipStream_t st = nullptr;
   ~nrpyell_mlp() {
     (void)hipFree(p); (void)hipFree(g); (void)hipFree(m); (void)hipFree(v); (void)hipFree(part);
@@ -773,12 +811,16 @@ struct nrpyell_mlp {
   }
   void release_seed() {
     (void)hipFree(seedX); (void)hipFree(seed_scale); (void)hipFree(seed_idx); (void)hipFree(seed_y);
-    seedX = nullptr; seed_scale = nullptr; seed_idx = nullptr; seed_y = nullptr;
+    (void)hipFree(seed_xx);
+    seedX = nullptr; seed_scale = nullptr; seed_idx = nullptr; seed_y = nullptr; seed_xx = nullptr;
     seed_cap = 0;
+    seed_nxx = 0;
   }
-  void ensure_seed(long rows) {
-    if (rows <= seed_cap) return;
+  void ensure_seed(long rows, int nxx) {
+    if (rows <= seed_cap && nxx <= seed_nxx) return;
     release_seed();  // a failed allocation below leaves seed_cap 0: the next seed allocates again
+    seed_xx = mlp_alloc<double>((size_t)nxx);
+    seed_nxx = nxx;
     seedX = mlp_alloc<bf16_t>((size_t)rows * MLP_K0);
     seed_scale = mlp_alloc<double>((size_t)rows);
     seed_idx = mlp_alloc<long>((size_t)rows);
@@ -861,6 +903,11 @@ struct nrpyell_mlp {
     w.n_params = n_params;
     w.part = part;
     hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(4 * WG_GROUPS + TR_SPLITS), dim3(256), 0, st, w);
+  }
+  // outputs of M feature rows (M a multiple of 64) on a stream
+  void forward(const bf16_t *X, long M, float *y, hipStream_t stream) {
+    hipLaunchKernelGGL(mlp_forward_fused_kernel, dim3((unsigned)((M + FI_R - 1) / FI_R)), dim3(256), 0, stream, X, pws,
+                       p, offsets(), copies(), M, y);
   }
   // g = the summed partials; with update, one Adam step at learning rate lr
   void reduce(int update, float lr) {
@@ -971,8 +1018,7 @@ static int check_rows(int M) {
 extern "C" int nrpyell_mlp_forward(nrpyell_mlp *s, const void *x, int M, float *y_out) {
   return api_call([&]() -> int {
     if (check_rows(M)) return NRPYELL_EINVAL;
-    hipLaunchKernelGGL(mlp_forward_fused_kernel, dim3((M + FI_R - 1) / FI_R), dim3(256), 0, s->st, (const bf16_t *)x,
-                       s->pws, s->p, s->offsets(), s->copies(), M, y_out);
+    s->forward((const bf16_t *)x, M, y_out, s->st);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->st));
     return NRPYELL_OK;
@@ -1076,19 +1122,24 @@ extern "C" long nrpyell_mlp_feature_rows(const griddata_struct *gd) {
   return (n + 63) / 64 * 64;
 }
 
+// The feature kernel on the default stream; xx is device memory for the G0 + G1 + G2 coordinates.
+static void launch_features(const griddata_struct *gd, const GridDims &g, double *xx, void *X, double *scale,
+                            long *idx) {
+  const long rows = nrpyell_mlp_feature_rows(gd);
+  std::vector<double> h(gd->xx[0], gd->xx[0] + g.G0);
+  h.insert(h.end(), gd->xx[1], gd->xx[1] + g.G1);
+  h.insert(h.end(), gd->xx[2], gd->xx[2] + g.G2);
+  HIPCHK(hipMemcpy(xx, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(features_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, 0, g,
+                     feature_params(&gd->params), xx, xx + g.G0, xx + g.G0 + g.G1, rows, (bf16_t *)X, scale, idx);
+}
+
 // Features (device BF16 [rows x 64], padding rows zero), per-row u scale and grid index.
 extern "C" int nrpyell_mlp_features(const griddata_struct *gd, void *X, double *scale, long *idx) {
   return api_call([&]() -> int {
     const GridDims g = dims_from_params(&gd->params);
-    const long n = (long)(g.G0 - NRPYELL_NG) * g.N1 * g.N2, rows = (n + 63) / 64 * 64;
-    DevBuf<double> b0(g.G0), b1(g.G1), b2(g.G2);
-    double *x0 = b0.p, *x1 = b1.p, *x2 = b2.p;
-    HIPCHK(hipMemcpy(x0, gd->xx[0], g.G0 * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(x1, gd->xx[1], g.G1 * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(x2, gd->xx[2], g.G2 * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(X, 0, rows * MLP_K0 * sizeof(bf16_t)));
-    hipLaunchKernelGGL(features_kernel, dim3((n + 255) / 256), dim3(256), 0, 0, g, feature_params(&gd->params), x0, x1,
-                       x2, (bf16_t *)X, scale, idx);
+    DevBuf<double> xx(g.G0 + g.G1 + g.G2);
+    launch_features(gd, g, xx.p, X, scale, idx);
     HIPCHK(hipGetLastError());
     HIPCHK(hipDeviceSynchronize());
     return NRPYELL_OK;
@@ -1118,33 +1169,26 @@ extern "C" int nrpyell_mlp_seed(nrpyell_mlp *s, griddata_struct *gd, int smooth_
       return NRPYELL_EINVAL;
     }
     const GridDims g = dims_from_params(&gd->params);
-    const long n = (long)(g.G0 - NRPYELL_NG) * g.N1 * g.N2, rows = (n + 63) / 64 * 64;
-    s->ensure_seed(rows);
-    bf16_t *X = s->seedX;
-    double *scale = s->seed_scale;
-    long *idx = s->seed_idx;
-    float *y = s->seed_y;
-    int rc = nrpyell_mlp_features(gd, X, scale, idx);
-    if (rc != NRPYELL_OK) return rc;
-    const int chunk = 1 << 18;  // rows per forward pass (multiple of 64)
-    for (long r0 = 0; r0 < rows; r0 += chunk) {
-      const int M = (int)((rows - r0) < chunk ? (rows - r0) : chunk);
-      if ((rc = nrpyell_mlp_forward(s, X + r0 * MLP_K0, M, y + r0)) != NRPYELL_OK) return rc;
-    }
-    double *yn = gd->gridfuncs.y_n_gfs, *tmp = gd->gridfuncs.k_odd_gfs;
-    hipLaunchKernelGGL(seed_state_kernel, dim3((n + 255) / 256), dim3(256), 0, 0, g, n, y, scale, idx,
-                       gd->params.eta_damping, yn);
-    const dim3 sg((g.G0 - NRPYELL_NG + 63) / 64, g.N1, g.N2);
-    for (int k = 0; k < smooth_passes; k++) {
-      hipLaunchKernelGGL(smooth_kernel<0>, sg, dim3(64), 0, 0, g, yn, tmp);
-      hipLaunchKernelGGL(smooth_kernel<1>, sg, dim3(64), 0, 0, g, tmp, yn);
-      hipLaunchKernelGGL(smooth_kernel<2>, sg, dim3(64), 0, 0, g, yn, tmp);
-      HIPCHK(hipMemcpyAsync(yn, tmp, sizeof(double) * g.ntot, hipMemcpyDeviceToDevice, 0));
-    }
-    if (smooth_passes > 0) {
-      launch_fill_ghost_planes<double>(g, yn, 1, 0);
-      hipLaunchKernelGGL(v_from_u_kernel, dim3((g.ntot + 255) / 256), dim3(256), 0, 0, g.ntot,
-                         gd->params.eta_damping, yn);
+    const long n = (long)(g.G0 - NRPYELL_NG) * g.N1 * g.N2, rows = nrpyell_mlp_feature_rows(gd);
+    s->ensure_seed(rows, g.G0 + g.G1 + g.G2);
+    launch_features(gd, g, s->seed_xx, s->seedX, s->seed_scale, s->seed_idx);
+    s->forward(s->seedX, rows, s->seed_y, 0);
+    const double eta = gd->params.eta_damping;
+    double *yn = gd->gridfuncs.y_n_gfs, *other = gd->gridfuncs.k_odd_gfs;
+    const dim3 sg((g.G0 - NRPYELL_NG + 63) / 64, g.N1, g.N2), pg((unsigned)((n + 255) / 256));
+    if (smooth_passes == 0) {
+      hipLaunchKernelGGL(seed_state_kernel<true>, pg, dim3(256), 0, 0, g, n, s->seed_y, s->seed_scale, s->seed_idx,
+                         eta, yn);
+    } else {
+      // u alternates between the two arrays so that the last pass writes y_n
+      double *from = smooth_passes % 2 ? other : yn, *to = smooth_passes % 2 ? yn : other;
+      hipLaunchKernelGGL(seed_state_kernel<false>, pg, dim3(256), 0, 0, g, n, s->seed_y, s->seed_scale, s->seed_idx,
+                         eta, from);
+      for (int k = 1; k < smooth_passes; k++) {
+        hipLaunchKernelGGL(smooth_kernel<false>, sg, dim3(64), 0, 0, g, eta, from, to);
+        std::swap(from, to);
+      }
+      hipLaunchKernelGGL(smooth_kernel<true>, sg, dim3(64), 0, 0, g, eta, from, to);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipDeviceSynchronize());
