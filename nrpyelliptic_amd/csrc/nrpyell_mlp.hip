@@ -62,14 +62,14 @@ __device__ __forceinline__ long draw_row(unsigned long long seed, int m, long N)
 // 1. mlp_train_rows_kernel: a block takes TR_R rows through the forward pass (activations in
 //    LDS, ping-pong), the output layer and the loss, then back through the data-gradient chain
 //    dZ_{l-1} = (dZ_l W_l) * silu'(Z_{l-1}). Every product is row-local, so nothing crosses
-//    blocks. silu'(z) of each layer stays in registers: the lane that produces z in the forward
-//    epilogue holds the same (row, column) entries of dZ in the backward one. H_l (l = 0..5)
-//    and dZ_l (l = 1..5) leave the block transposed ([width x M], rows contiguous), which is the
-//    layout the weight gradients consume as MFMA operands.
-// 2. mlp_wgrad_kernel: dW_l = dZ_l^T H_{l-1}, db_l = column sums of dZ_l, and the output layer's
-//    gradients, over TR_SPLITS row ranges; each range writes its own partial (no atomics).
-// 3. mlp_adam_kernel: g = the partials summed in range order (deterministic), Adam, and the BF16
-//    weight copies (W_l and, for l >= 2, W_l transposed, the data-gradient chain's operand).
+//    blocks. silu'(z) stays with the lane that produces z in the forward epilogue: it holds the
+//    same (row, column) entries of dZ in the backward one. H_l (l = 0..5) and dZ_l (l = 1..5)
+//    leave the block transposed ([width x M], rows contiguous), which is the layout the weight
+//    gradients consume as MFMA operands.
+// 2. mlp_grad_kernel, mlp_small_kernel: dW_l = dZ_l^T H_{l-1}, db_l = column sums of dZ_l, and the output layer's
+//    gradients, as sums over TR_SPLITS row ranges in range order (deterministic), then Adam and
+//    the BF16 weight copies (W_l and, for l >= 2, W_l transposed, the data-gradient chain's
+//    operand).
 //
 // Arithmetic per entry matches the network definition: FP32 accumulation of BF16 products in
 // ascending inner index, z = acc + b, h = bf16(silu(z)), y = sum_k h_k w_k + b (FP32),
@@ -79,9 +79,6 @@ constexpr int TR_R = 32;        // rows per block
 constexpr int TR_WAVES = 8;     // wave w owns columns 32w .. 32w+31 of every 256-wide layer
 constexpr int TR_LD = MLP_W + 8;
 constexpr int TR_SPLITS = 32;   // row ranges of the weight-gradient reduction
-constexpr int WG_GROUPS = MLP_HIDDEN * TR_SPLITS;  // (layer, row range) groups of the weight gradients
-constexpr int TR_LDS_DSL = 3;         // layers whose silu'(z) the row kernel keeps in LDS
-constexpr int WG_G = 2;               // inner steps per load group of the weight-gradient kernel
 
 // Operand layout of a matrix X[rows][inner] (rows a multiple of 32, inner a multiple of 16):
 // lane (li, lj) of a wave feeds the 32x32x16 MFMA for rows 32 t .. 32 t + 31 and inner step q
@@ -117,78 +114,63 @@ struct TrainArgs {
   double *loss;                    // += sum over the block's rows of (y - t)^2 / M
 };
 
-// rows r0 .. r0+31 of an LDS tile (width WD) -> the transposed global [WD x M] in the operand
-// layout (rows = the WD columns, inner = minibatch rows)
-template <int WD>
-__device__ __forceinline__ void store_transposed(const bf16_t *buf, bf16_t *__restrict__ out, int r0, int M, int tid) {
-  constexpr int PER = TR_R * WD / (64 * TR_WAVES);  // rows per thread: 16 (WD 256) or 4 (WD 64)
-  const int c = tid % WD, q = tid / WD;
-  const int m = r0 + PER * q, M16 = M / 16;
-  bf16_t v[PER];
+// The 32 x 32 MFMA tile of columns 32 ct .. and the block's rows r0 .. r0+31 to the transposed
+// global [width x M] in the operand layout (rows = columns of the layer, inner = minibatch rows),
+// straight from the accumulators' layout: v[g] holds column li, rows 8 g + 4 lj .. + 3, half of an
+// 8-element chunk; lanes lj = 0, 1 fill it, so a wave's store is 512 consecutive bytes.
+__device__ __forceinline__ void store_tile_transposed(const bf16x4 (&v)[4], bf16_t *__restrict__ out, int ct, int r0,
+                                                      int M, int li, int lj) {
+  bf16_t *o = out + ((long)(ct * (M / 16) + r0 / 16) * 64 + li) * 8 + 4 * lj;
 #pragma unroll
-  for (int i = 0; i < PER; i++) v[i] = buf[(PER * q + i) * TR_LD + c];
-  if (PER == 16) {
-    bf16x8 lo, hi;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      lo[i] = v[i];
-      hi[i] = v[8 + i];
-    }
-    *(bf16x8 *)(out + swz(c, m, M16)) = lo;
-    *(bf16x8 *)(out + swz(c, m + 8, M16)) = hi;
-  } else {
-    bf16_t *o = out + swz(c, m, M16);
-#pragma unroll
-    for (int i = 0; i < PER; i++) o[i] = v[i];
-  }
+  for (int g = 0; g < 4; g++) *(bf16x4 *)(o + ((g >> 1) * 64 + (g & 1) * 32) * 8) = v[g];
 }
 
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = sigmoidf_(z);
-  return s * (1.0f + z * (1.0f - s));
-}
-
+// 256 blocks at the production minibatch of 8192 rows, one per CU: each of the ten dependent
+// products is 16 MFMAs of latency behind 128 KB of weights from L2, so what counts is the work
+// between them. silu' of four layers stays in registers (of all five it does not fit 256), the
+// transposed copies go to memory from the accumulators, and the sigmoid has no division: 28.0 us
+// (silu' of three layers in LDS, the copies read back from the LDS tiles, divisions: 31.1 us).
 __global__ void __launch_bounds__(512) mlp_train_rows_kernel(TrainArgs a) {
   __shared__ __attribute__((aligned(16))) bf16_t Hb[2][TR_R * TR_LD];
   __shared__ float s_part[TR_WAVES][TR_R];
   __shared__ float s_t[TR_R], s_dy[TR_R];
-  __shared__ long s_row[TR_R];
-  // silu'(z) of layers 1..TR_LDS_DSL, each thread's 16 entries at [layer][r][thread] (read back by
-  // the same thread); layers above stay in registers
-  __shared__ float s_dsl[TR_LDS_DSL][16][64 * TR_WAVES];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ float s_dsl[16][64 * TR_WAVES];  // silu' of layer 1, read back by the thread that wrote it
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, lj = lane >> 5;
   const int r0 = blockIdx.x * TR_R;
   // this lane's column of every 256-wide layer; the eight 32-column slices are rotated by the
   // block index so that concurrent blocks read different weight rows (no change to any sum)
   const int ct = (wave + blockIdx.x) & (TR_WAVES - 1);
   const int c = ct * 32 + li;
-  if (tid < TR_R) {
-    const long row = a.gather ? draw_row(a.seed, r0 + tid, a.N) : (long)(r0 + tid);
-    s_row[tid] = row;
-    s_t[tid] = a.t[row];
-  }
-  __syncthreads();
-  if (tid < TR_R * 8) {  // 32 rows x 64 BF16 features = 256 chunks of 16 B
-    const int row = tid >> 3, ch = tid & 7;
-    *(bf16x8 *)(&Hb[0][row * TR_LD + 8 * ch]) = *(const bf16x8 *)(a.X + s_row[row] * MLP_K0 + 8 * ch);
-  }
-  __syncthreads();
-  store_transposed<MLP_K0>(Hb[0], a.Ht[0], r0, a.M, tid);
-  // accumulator r of lane (li, lj): row 8*(r/4) + 4*lj + r%4 of the block, column c
-  float dsl[MLP_HIDDEN][16];
   // the weight operands of the next product are loaded (all of them, 16 B per lane per
   // 16-wide inner step) as soon as the current product's MFMAs are issued, so their latency
-  // overlaps the epilogue, the barrier and the transposed store
+  // overlaps the epilogue and the barrier
   bf16x8 bv[MLP_W / 16];
 #pragma unroll
   for (int q = 0; q < MLP_K0 / 16; q++)
     bv[q] = *(const bf16x8 *)(a.pws + a.wc.fs[1] + ((long)ct * (MLP_K0 / 16) + q) * 512 + 8 * lane);
+  if (tid < TR_R * 8) {  // 32 rows x 64 BF16 features = 256 chunks of 16 B
+    const int row = tid >> 3, ch = tid & 7;
+    const long src = a.gather ? draw_row(a.seed, r0 + row, a.N) : (long)(r0 + row);
+    if (ch == 0) s_t[row] = a.t[src];
+    *(bf16x8 *)(&Hb[0][row * TR_LD + 8 * ch]) = *(const bf16x8 *)(a.X + src * MLP_K0 + 8 * ch);
+  }
+  __syncthreads();
+  {  // H_0 transposed: 4 rows of one column per thread
+    const int col = tid % MLP_K0, m = 4 * (tid / MLP_K0);
+    bf16x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = Hb[0][(m + i) * TR_LD + col];
+    *(bf16x4 *)(a.Ht[0] + swz(col, r0 + m, a.M / 16)) = v;
+  }
+  // accumulator r of lane (li, lj): row 8*(r/4) + 4*lj + r%4 of the block, column c
+  float dsl[MLP_HIDDEN][16];  // silu'(z); layer 1's waits in s_dsl
   int cur = 0;
 #pragma unroll
   for (int l = 1; l <= MLP_HIDDEN; l++) {
     const int Kl = l == 1 ? MLP_K0 : MLP_W;
     const bf16_t *Hin = Hb[cur] + li * TR_LD + 8 * lj;
+    const float bc = a.p[a.off.b[l] + c];
     floatx16 acc;
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
@@ -200,31 +182,43 @@ __global__ void __launch_bounds__(512) mlp_train_rows_kernel(TrainArgs a) {
     const bf16_t *Wn = a.pws + (l < MLP_HIDDEN ? a.wc.fs[l + 1] : a.wc.ts[MLP_HIDDEN]) + (long)ct * 16 * 512 + 8 * lane;
 #pragma unroll
     for (int q = 0; q < MLP_W / 16; q++) bv[q] = *(const bf16x8 *)(Wn + 512 * q);
-    bf16_t *Hout = Hb[cur ^ 1];
-    const float bc = a.p[a.off.b[l] + c];
+    __builtin_amdgcn_sched_barrier(0);
+    bf16_t *Hout = Hb[cur ^ 1] + 4 * lj * TR_LD + c;
+    bf16x4 hb[4];
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int row = 8 * (r >> 2) + 4 * lj + (r & 3);
-      const float z = acc[r] + bc;
-      if (l <= TR_LDS_DSL)
-        s_dsl[l - 1][r][tid] = dsilu(z);
-      else
-        dsl[l - 1][r] = dsilu(z);
-      Hout[row * TR_LD + c] = to_bf16(z * sigmoidf_(z));
+    for (int g = 0; g < 4; g++) {
+      floatx4 h;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float z = acc[4 * g + i] + bc, s = sigmoidf_(z);
+        const float ds = s * (1.0f + z * (1.0f - s));
+        if (l == 1)
+          s_dsl[4 * g + i][tid] = ds;
+        else
+          dsl[l - 1][4 * g + i] = ds;
+        h[i] = z * s;
+      }
+      hb[g] = __builtin_convertvector(h, bf16x4);
+#pragma unroll
+      for (int i = 0; i < 4; i++) Hout[(8 * g + i) * TR_LD] = hb[g][i];
     }
     __syncthreads();
+    store_tile_transposed(hb, a.Ht[l], ct, r0, a.M, li, lj);
     cur ^= 1;
-    store_transposed<MLP_W>(Hb[cur], a.Ht[l], r0, a.M, tid);
   }
   // output layer: wave w sums columns 32w .. 32w+31 of every row, then the 8 partials in a fixed order
   const float *wout = a.p + a.off.w[MLP_HIDDEN + 1];
   if (lane < TR_R) {
-    const bf16_t *h = Hb[cur] + lane * TR_LD + wave * 32;
     float acc = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < 32; k++) acc += (float)h[k] * wout[wave * 32 + k];
+#pragma unroll
+    for (int k = 0; k < 32; k += 8) {
+      const bf16x8 h = *(const bf16x8 *)(Hb[cur] + lane * TR_LD + wave * 32 + k);
+#pragma unroll
+      for (int i = 0; i < 8; i++) acc += (float)h[i] * wout[wave * 32 + k + i];
+    }
     s_part[wave][lane] = acc;
   }
+  const float wc_ = wout[c];
   __syncthreads();
   if (tid < 64) {
     double l2 = 0.0;
@@ -242,187 +236,313 @@ __global__ void __launch_bounds__(512) mlp_train_rows_kernel(TrainArgs a) {
     if (tid == 0) atomicAdd(a.loss, l2);
   }
   __syncthreads();
-  // dZ_5 into the other buffer (H_4 there is no longer read)
-  {
-    bf16_t *D = Hb[cur ^ 1];
-    const float wc_ = wout[c];
+  // dZ_5 into the other buffer (H_4 there is no longer read), then dZ_{l-1} = (dZ_l W_l) *
+  // silu'(Z_{l-1}), l = 5..2: A = dZ_l (LDS), B(k, n) = W_l^T[k][n]
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int row = 8 * (r >> 2) + 4 * lj + (r & 3);
-      D[row * TR_LD + c] = to_bf16(s_dy[row] * wc_ * dsl[MLP_HIDDEN - 1][r]);
-    }
-  }
-  __syncthreads();
-  cur ^= 1;
-  store_transposed<MLP_W>(Hb[cur], a.dZt[MLP_HIDDEN], r0, a.M, tid);
-  // dZ_{l-1} = (dZ_l W_l) * silu'(Z_{l-1}), l = 5..2: A = dZ_l (LDS), B(k, n) = W_l^T[k][n]
-#pragma unroll
-  for (int l = MLP_HIDDEN; l >= 2; l--) {
-    const bf16_t *Din = Hb[cur] + li * TR_LD + 8 * lj;
+  for (int l = MLP_HIDDEN + 1; l >= 2; l--) {
     floatx16 acc;
+    if (l > MLP_HIDDEN) {
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+      for (int r = 0; r < 16; r++) acc[r] = s_dy[8 * (r >> 2) + 4 * lj + (r & 3)] * wc_;
+    } else {
+      const bf16_t *Din = Hb[cur] + li * TR_LD + 8 * lj;
 #pragma unroll
-    for (int q = 0; q < MLP_W / 16; q++)
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(Din + 16 * q), bv[q], acc, 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    if (l > 2) {
-      const bf16_t *WT = a.pws + a.wc.ts[l - 1] + (long)ct * 16 * 512 + 8 * lane;
+      for (int r = 0; r < 16; r++) acc[r] = 0.0f;
 #pragma unroll
-      for (int q = 0; q < MLP_W / 16; q++) bv[q] = *(const bf16x8 *)(WT + 512 * q);
+      for (int q = 0; q < MLP_W / 16; q++)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(Din + 16 * q), bv[q], acc, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (l > 2) {
+        const bf16_t *WT = a.pws + a.wc.ts[l - 1] + (long)ct * 16 * 512 + 8 * lane;
+#pragma unroll
+        for (int q = 0; q < MLP_W / 16; q++) bv[q] = *(const bf16x8 *)(WT + 512 * q);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    bf16_t *Dout = Hb[cur ^ 1];
+    bf16_t *Dout = Hb[cur ^ 1] + 4 * lj * TR_LD + c;
+    bf16x4 db[4];
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int row = 8 * (r >> 2) + 4 * lj + (r & 3);
-      Dout[row * TR_LD + c] = to_bf16(acc[r] * (l - 1 <= TR_LDS_DSL ? s_dsl[l - 2][r][tid] : dsl[l - 2][r]));
+    for (int g = 0; g < 4; g++) {
+      floatx4 d;
+#pragma unroll
+      for (int i = 0; i < 4; i++) d[i] = acc[4 * g + i] * (l == 2 ? s_dsl[4 * g + i][tid] : dsl[l - 2][4 * g + i]);
+      db[g] = __builtin_convertvector(d, bf16x4);
+      if (l > 2) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) Dout[(8 * g + i) * TR_LD] = db[g][i];
+      }
     }
-    __syncthreads();
+    if (l > 2) __syncthreads();
+    store_tile_transposed(db, a.dZt[l - 1], ct, r0, a.M, li, lj);
     cur ^= 1;
-    store_transposed<MLP_W>(Hb[cur], a.dZt[l - 1], r0, a.M, tid);
   }
 }
 
-struct WgradArgs {
+// The BF16 copies of parameter k (see WeightCopies).
+__device__ __forceinline__ void store_weight(const WeightCopies &wc, long k, float v, bf16_t *__restrict__ pws) {
+  const bf16_t b = to_bf16(v);
+#pragma unroll
+  for (int l = 1; l <= MLP_HIDDEN; l++) {
+    const int Kl = l == 1 ? MLP_K0 : MLP_W;
+    const long d = k - wc.w_off[l];
+    if (d >= 0 && d < (long)MLP_W * Kl) {
+      const int n = (int)(d / Kl), kk = (int)(d % Kl);
+      pws[wc.fs[l] + swz(n, kk, Kl / 16)] = b;
+      if (l >= 2) pws[wc.ts[l] + swz(kk, n, MLP_W / 16)] = b;
+    }
+  }
+}
+
+__global__ void refresh_weights_kernel(long n, const float *__restrict__ p, WeightCopies wc,
+                                       bf16_t *__restrict__ pws) {
+  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) store_weight(wc, k, p[k], pws);
+}
+
+// Adam on one parameter, in the state arrays p, mo (first moment), ve (second); c1, c2 the bias
+// corrections 1 - beta^t.
+struct AdamArgs {
+  float *p, *mo, *ve;
+  bf16_t *pws;
+  float lr, c1, c2;
+  WeightCopies wc;
+};
+__device__ __forceinline__ void adam_update(const AdamArgs &o, long k, float gk) {
+  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  const float m = b1 * o.mo[k] + (1.0f - b1) * gk;
+  const float v = b2 * o.ve[k] + (1.0f - b2) * gk * gk;
+  o.mo[k] = m;
+  o.ve[k] = v;
+  const float pk = o.p[k] - o.lr * (m / o.c1) / (sqrtf(v / o.c2) + eps);
+  o.p[k] = pk;
+  store_weight(o.wc, k, pk, o.pws);
+}
+
+struct GradArgs {
   const bf16_t *Ht[MLP_HIDDEN + 1];
   const bf16_t *dZt[MLP_HIDDEN + 1];
   const float *dy;
   int M, chunk;  // rows per range (multiple of 16)
   MlpOffsets off;
-  long n_params;
-  float *part;   // [TR_SPLITS x n_params]
+  float *g;      // [n_params]
+  float *part;   // [TR_SPLITS x GR_PART]: layer 1 and the output layer by ranges
+  int update;    // 1: also an Adam step
+  AdamArgs adam;
 };
 
-// One wave's (32 NT) x (32 KT) block of C[n][k] = sum_{m in [m0, m1)} A[n][m] B[k][m] for the
-// rows n = 32 ta .., k = 32 tb .. of two transposed minibatch arrays in the operand layout (inner
-// = the M minibatch rows), loaded straight from global as MFMA operands (1 KB per wave and load)
-// in groups of WG_G 16-row inner steps, double-buffered (the loads of group g+1 are in flight
-// while group g's MFMAs run). C goes to G (row stride ldg); with gb != null the row sums of A
-// (bias gradient) go to gb.
-template <int NT, int KT>
-__device__ __forceinline__ void wgrad_block(const bf16_t *__restrict__ A, int ta, const bf16_t *__restrict__ B, int tb,
-                                            int M, int m0, int m1, float *__restrict__ G, int ldg,
-                                            float *__restrict__ gb) {
-  const int lane = threadIdx.x & 63, li = lane & 31, lj = lane >> 5;
-  const long M16 = M / 16;
-  const bf16_t *Ap[NT], *Bp[KT];
+// The partials of one range: dW_1 as 16 tiles of 32 x 32, db_1, the output layer's weights and bias.
+constexpr int GR_PB1 = MLP_W * MLP_K0, GR_PW = GR_PB1 + MLP_W, GR_PB = GR_PW + MLP_W, GR_PART = GR_PB + 1;
+
+__device__ __forceinline__ void finish_gradient(const GradArgs &a, long k, float gk) {
+  a.g[k] = gk;
+  if (a.update) adam_update(a.adam, k, gk);
+}
+
+// 2. The gradients of one minibatch and the Adam step on them. A gradient is the sum over TR_SPLITS
+// row ranges, in range order, of FP32 partials: dW_l = dZ_l^T H_{l-1} by MFMA in ascending rows,
+// db_l the column sums of dZ_l, the output layer's by rows.
+//
+// Layers 2..5: block b owns one 32 x 32 tile of a dW_l through all ranges. Its eight waves take four
+// ranges each, the partials meet in LDS (132 KB) and every thread adds the 32 of its two entries. So
+// no partial leaves the chip (as global arrays they were 36 MB written and read again). A tile costs its reads of dZ_l and H_{l-1}, 1 MB at 8192 rows, and L1's rate sets the
+// kernel's time: 256 tiles, one per CU, is the split with the least per CU. GR_D inner steps of 16
+// rows are in flight per wave, across the ranges' ends. XCD x (where workgroups with b % 8 = x
+// run) has half the rows of one layer, so its L2 serves their reuse.
+// Layer 1 and the output layer would be a second block on a few CUs, which doubles the time;
+// instead a ninth wave of every block takes a share of their ranges, and mlp_small_kernel adds
+// those partials (2 MB). 8192 rows: 23.6 us and 4.8 us (gradients by row ranges 20.4 us, then
+// reduction and Adam 9.8 us).
+constexpr int GR_D = 8;
+constexpr int GR_BLOCKS = 8 * (MLP_W / 32) * (MLP_HIDDEN - 1);
+constexpr int GR_THREADS = 9 * 64;
+static_assert(GR_BLOCKS == 8 * TR_SPLITS, "the ninth waves cover every range of layer 1 and the output layer");
+
+// GR_D inner steps of a pair of operand tiles from step t on, at a uniform address. A group that
+// starts past the last row reads the end of the tile's rows and the arrays' padding: not used.
+struct GradRing {
+  bf16x8 a[GR_D], b[GR_D];
+};
+__device__ __forceinline__ void grad_load(GradRing &r, int i, const bf16_t *A, const bf16_t *B, int t, int M16) {
+  const long o = (long)min(t, M16) * 512;
+  const unsigned v = 16 * (threadIdx.x & 63) + 1024 * i;
+  r.a[i] = *(const bf16x8 *)((const char *)(A + o) + v);
+  r.b[i] = *(const bf16x8 *)((const char *)(B + o) + v);
+}
+__device__ __forceinline__ void grad_fill(GradRing &r, const bf16_t *A, const bf16_t *B, int t, int M16) {
 #pragma unroll
-  for (int x = 0; x < NT; x++) Ap[x] = A + ((ta + x) * M16 * 64 + lane) * 8;
+  for (int i = 0; i < GR_D; i++) {
+    grad_load(r, i, A, B, t, M16);
+    __builtin_amdgcn_sched_barrier(0);  // issued in the order of use: a wait for one leaves the later ones in flight
+  }
+}
+// One range of a tile: its cs steps from s0 on (ns of them real), the group of (A1, B1) at `then`
+// loaded as the last one is used; acc += A B^T, bsum += this lane's elements of A where `bias`.
+__device__ __forceinline__ void grad_range(GradRing &r, const bf16_t *A, const bf16_t *B, int s0, int cs, int ns,
+                                           const bf16_t *A1, const bf16_t *B1, int then, int M16, bool bias,
+                                           floatx16 &acc, float &bsum) {
+  for (int q0 = 0; q0 < cs; q0 += GR_D) {
+    const bool more = q0 + GR_D < cs;
+    const int next = more ? s0 + q0 + GR_D : then;
+    const bf16_t *An = more ? A : A1, *Bn = more ? B : B1;
 #pragma unroll
-  for (int y = 0; y < KT; y++) Bp[y] = B + ((tb + y) * M16 * 64 + lane) * 8;
-  floatx16 acc[NT][KT];
-#pragma unroll
-  for (int x = 0; x < NT; x++)
-#pragma unroll
-    for (int y = 0; y < KT; y++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[x][y][r] = 0.0f;
-  float bsum[NT];
-#pragma unroll
-  for (int x = 0; x < NT; x++) bsum[x] = 0.0f;
-  const bool bias = gb != nullptr;
-  const int nsteps = m1 > m0 ? (m1 - m0) / 16 : 0;
-  const int ngroups = (nsteps + WG_G - 1) / WG_G;
-  bf16x8 a0[WG_G][NT], b0[WG_G][KT], a1[WG_G][NT], b1[WG_G][KT];
-  auto load = [&](bf16x8 (*av)[NT], bf16x8 (*bw)[KT], int g) {
-#pragma unroll
-    for (int q = 0; q < WG_G; q++)
-      if (g * WG_G + q < nsteps) {
-        const long o = (long)(m0 / 16 + g * WG_G + q) * 512;  // inner step m / 16
-#pragma unroll
-        for (int x = 0; x < NT; x++) av[q][x] = *(const bf16x8 *)(Ap[x] + o);
-#pragma unroll
-        for (int y = 0; y < KT; y++) bw[q][y] = *(const bf16x8 *)(Bp[y] + o);
-      }
-  };
-  auto mma = [&](bf16x8 (*av)[NT], bf16x8 (*bw)[KT], int g) {
-#pragma unroll
-    for (int q = 0; q < WG_G; q++)
-      if (g * WG_G + q < nsteps) {
-#pragma unroll
-        for (int x = 0; x < NT; x++)
-#pragma unroll
-          for (int y = 0; y < KT; y++)
-            acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[q][x], bw[q][y], acc[x][y], 0, 0, 0);
+    for (int i = 0; i < GR_D; i++) {
+      if (q0 + i < ns) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(r.a[i], r.b[i], acc, 0, 0, 0);
         if (bias) {
 #pragma unroll
-          for (int x = 0; x < NT; x++)
-#pragma unroll
-            for (int i = 0; i < 8; i++) bsum[x] += (float)av[q][x][i];
+          for (int e = 0; e < 8; e++) bsum += (float)r.a[i][e];
         }
       }
-  };
-  if (ngroups > 0) load(a0, b0, 0);
-  for (int g = 0; g < ngroups; g += 2) {
-    if (g + 1 < ngroups) load(a1, b1, g + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(a0, b0, g);
-    __builtin_amdgcn_sched_barrier(0);
-    if (g + 2 < ngroups) load(a0, b0, g + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    if (g + 1 < ngroups) mma(a1, b1, g + 1);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  // accumulator r of lane (li, lj) is row 8*(r/4) + 4*lj + r%4, column li of its 32 x 32 tile
-#pragma unroll
-  for (int x = 0; x < NT; x++)
-#pragma unroll
-    for (int y = 0; y < KT; y++)
-#pragma unroll
-      for (int r = 0; r < 16; r++)
-        G[(long)(32 * x + 8 * (r >> 2) + 4 * lj + (r & 3)) * ldg + 32 * y + li] = acc[x][y][r];
-  if (bias) {
-#pragma unroll
-    for (int x = 0; x < NT; x++) {
-      const float t = bsum[x] + __shfl_xor(bsum[x], 32, 64);
-      if (lj == 0) gb[32 * x + li] = t;
+      grad_load(r, i, An, Bn, next, M16);
     }
   }
 }
-
-// Weight gradients over row ranges. Blocks 0 .. 4*WG_GROUPS-1: group (layer l, range s) has four
-// blocks nt = 0..3, each the 64 rows 64 nt .. 64 nt + 63 of dW_l (all K_l columns): for l >= 2
-// wave w takes columns 64 w .. 64 w + 63 (2 x 2 MFMA tiles), for l = 1 wave w the 32 x 32
-// quarter (w / 2, w % 2) of the 64 x 64 block. Block b = 32 (g / 8) + 8 nt + g % 8 for group g,
-// so the four blocks of a group share b mod 8, i.e. one XCD (workgroups are dealt to the XCDs
-// round-robin) and one L2, where the group's dZ_l and H_{l-1} row slices are reused. The last
-// TR_SPLITS blocks: the output layer's gradients, one range each.
-__global__ void __launch_bounds__(256) mlp_wgrad_kernel(WgradArgs a) {
-  const int tid = threadIdx.x, wave = tid >> 6;
-  const int b = blockIdx.x;
-  if (b >= 4 * WG_GROUPS) {
-    const int s = b - 4 * WG_GROUPS;
-    const int m0 = s * a.chunk, m1 = min(a.M, m0 + a.chunk);
-    float *P = a.part + (long)s * a.n_params;
-    // gw[k] = sum_m dy[m] H_5[m][k], gb = sum_m dy[m]; thread k reads row k of H_5^T (operand layout)
-    const bf16_t *h = a.Ht[MLP_HIDDEN] + (((long)(tid >> 5) * (a.M / 16)) * 64 + (tid & 31)) * 8;
-    float acc = 0.0f, accb = 0.0f;
-    for (int m = m0; m < m1; m += 8) {
-      const bf16x8 hv = *(const bf16x8 *)(h + ((long)(m >> 4) * 64 + ((m >> 3) & 1) * 32) * 8);
+// accumulator r of lane (li, lj) is row 8*(r/4) + 4*lj + r%4, column li of the 32 x 32 tile
+__device__ __forceinline__ void store_tile(float *P, const floatx16 &acc, int li, int lj) {
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        acc += a.dy[m + i] * (float)hv[i];
-        accb += a.dy[m + i];
+  for (int r = 0; r < 16; r++) P[(8 * (r >> 2) + 4 * lj + (r & 3)) * 32 + li] = acc[r];
+}
+
+// The ninth wave of block b: two tiles of dW_1 for one range, and for b < 4 TR_SPLITS 64 of the output
+// layer's inputs for one range.
+__device__ __forceinline__ void grad_small_layers(const GradArgs &a, int b, int nrange, int M16, int cs) {
+  const int lane = threadIdx.x & 63, li = lane & 31, lj = lane >> 5;
+  const int s = b >> 3, t0 = (2 * b) & 15;  // tiles t0, t0 + 1: the same 32 rows n, both column halves
+  if (s < nrange) {
+    GradRing ring;
+    const bf16_t *A = a.dZt[1] + (long)(t0 >> 1) * M16 * 512, *B = a.Ht[0], *B1 = B + (long)M16 * 512;
+    float *P = a.part + (long)s * GR_PART;
+    grad_fill(ring, A, B, s * cs, M16);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      floatx16 acc;
+      float bsum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+      grad_range(ring, A, u == 0 ? B : B1, s * cs, cs, min(cs, M16 - s * cs), A, B1, u == 0 ? s * cs : M16, M16, u == 0,
+                 acc, bsum);
+      store_tile(P + 1024 * (t0 + u), acc, li, lj);
+      bsum += __shfl_xor(bsum, 32, 64);
+      if (u == 0 && lj == 0) P[GR_PB1 + 32 * (t0 >> 1) + li] = bsum;
+    }
+  }
+  const int so = b >> 2, q = b & 3;
+  if (b < 4 * TR_SPLITS && so < nrange) {
+    // gw[k] = sum_m dy[m] H_5[m][k], gb = sum_m dy[m]; a lane reads one row k of H_5^T, GR_D chunks of
+    // 8 rows in flight
+    const bf16_t *h = a.Ht[MLP_HIDDEN] + ((long)(2 * q + lj) * M16 * 64 + li) * 8;
+    const int m1 = min(a.M, (so + 1) * a.chunk);
+    float gw = 0.0f, gb = 0.0f;
+    for (int m = so * a.chunk; m < m1; m += 8 * GR_D) {
+      bf16x8 hv[GR_D];
+      floatx4 dv[GR_D][2];
+#pragma unroll
+      for (int u = 0; u < GR_D; u++) {
+        const int c = min(m + 8 * u, m1 - 8);
+        hv[u] = *(const bf16x8 *)(h + ((long)(c >> 4) * 64 + ((c >> 3) & 1) * 32) * 8);
+        dv[u][0] = *(const floatx4 *)(a.dy + c);
+        dv[u][1] = *(const floatx4 *)(a.dy + c + 4);
+      }
+#pragma unroll
+      for (int u = 0; u < GR_D; u++)
+        if (m + 8 * u < m1) {
+#pragma unroll
+          for (int i = 0; i < 8; i++) {
+            const float d = dv[u][i >> 2][i & 3];
+            gw += d * (float)hv[u][i];
+            gb += d;
+          }
+        }
+    }
+    a.part[(long)so * GR_PART + GR_PW + 64 * q + lane] = gw;
+    if (q == 0 && lane == 0) a.part[(long)so * GR_PART + GR_PB] = gb;
+  }
+}
+
+__global__ void __launch_bounds__(GR_THREADS) mlp_grad_kernel(GradArgs a) {
+  __shared__ float s_p[TR_SPLITS][32 * 32];
+  __shared__ float s_b[TR_SPLITS][32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, lj = lane >> 5;
+  const int b = blockIdx.x;
+  const int nrange = (a.M + a.chunk - 1) / a.chunk;  // ranges with rows; the others add zero
+  const int M16 = a.M / 16, cs = a.chunk / 16;       // inner steps: in all, per range
+  const int x = b & 7, j = b >> 3;
+  const int l = 2 + (x >> 1), nt = 4 * (x & 1) + (j >> 3), kt = j & 7;
+  if (wave == 8) {
+    grad_small_layers(a, b, nrange, M16, cs);
+  } else {
+    const bf16_t *A = a.dZt[l] + (long)nt * M16 * 512, *B = a.Ht[l - 1] + (long)kt * M16 * 512;
+    GradRing ring;
+    grad_fill(ring, A, B, wave * cs, M16);
+    // this wave's ranges wave, wave + 8, ..: one accumulator each, so the waves run free of each other
+    // until every range is done
+    constexpr int NPH = TR_SPLITS / 8;
+    floatx16 acc[NPH];
+    float bsum[NPH];
+#pragma unroll
+    for (int ph = 0; ph < NPH; ph++) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[ph][r] = 0.0f;
+      bsum[ph] = 0.0f;
+      const int s0 = (8 * ph + wave) * cs;
+      if (8 * ph < nrange)
+        grad_range(ring, A, B, s0, cs, min(cs, M16 - s0), A, B, s0 + 8 * cs, M16, kt == 0, acc[ph], bsum[ph]);
+    }
+#pragma unroll
+    for (int ph = 0; ph < NPH; ph++) {
+      store_tile(s_p[8 * ph + wave], acc[ph], li, lj);
+      if (kt == 0) {
+        const float t = bsum[ph] + __shfl_xor(bsum[ph], 32, 64);
+        if (lj == 0) s_b[8 * ph + wave][li] = t;
       }
     }
-    P[a.off.w[MLP_HIDDEN + 1] + tid] = acc;
-    if (tid == 0) P[a.off.b[MLP_HIDDEN + 1]] = accb;
-    return;
   }
-  const int q = b >> 5, rem = b & 31, nt = rem >> 3, g = q * 8 + (rem & 7);
-  const int l = 1 + g / TR_SPLITS, s = g % TR_SPLITS;
-  const int m0 = s * a.chunk, m1 = min(a.M, m0 + a.chunk);
-  float *P = a.part + (long)s * a.n_params;
-  if (l == 1) {
-    const int n0 = nt * 64 + (wave >> 1) * 32, k0 = (wave & 1) * 32;
-    wgrad_block<1, 1>(a.dZt[1], n0 / 32, a.Ht[0], k0 / 32, a.M, m0, m1,
-                      P + a.off.w[1] + (long)n0 * MLP_K0 + k0, MLP_K0,
-                      (wave & 1) == 0 ? P + a.off.b[1] + n0 : nullptr);
+  __syncthreads();
+  if (tid >= 512) return;
+  float gw[2] = {0.0f, 0.0f}, gb = 0.0f;
+#pragma unroll
+  for (int s = 0; s < TR_SPLITS; s++) {
+#pragma unroll
+    for (int e = 0; e < 2; e++) gw[e] += s_p[s][tid + 512 * e];
+  }
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const int k = tid + 512 * e;
+    finish_gradient(a, a.off.w[l] + (long)(32 * nt + (k >> 5)) * MLP_W + 32 * kt + (k & 31), gw[e]);
+  }
+  if (kt == 0 && tid < 32) {
+    for (int s = 0; s < TR_SPLITS; s++) gb += s_b[s][tid];
+    finish_gradient(a, a.off.b[l] + 32 * nt + tid, gb);
+  }
+}
+
+// Layer 1 and the output layer: the ranges' partials of mlp_grad_kernel in range order, Adam.
+__global__ void __launch_bounds__(256) mlp_small_kernel(GradArgs a) {
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  if (j >= GR_PART) return;
+  const int nrange = (a.M + a.chunk - 1) / a.chunk;
+  float v[TR_SPLITS], gk = 0.0f;
+#pragma unroll
+  for (int s = 0; s < TR_SPLITS; s++) v[s] = s < nrange ? a.part[(long)s * GR_PART + j] : 0.0f;
+#pragma unroll
+  for (int s = 0; s < TR_SPLITS; s++) gk += v[s];
+  long k;
+  if (j < GR_PB1) {
+    const int t = j >> 10, e = j & 1023;
+    k = a.off.w[1] + (32 * (t >> 1) + (e >> 5)) * MLP_K0 + 32 * (t & 1) + (e & 31);
+  } else if (j < GR_PW) {
+    k = a.off.b[1] + (j - GR_PB1);
   } else {
-    const int n0 = nt * 64, k0 = wave * 64;
-    wgrad_block<2, 2>(a.dZt[l], n0 / 32, a.Ht[l - 1], k0 / 32, a.M, m0, m1,
-                      P + a.off.w[l] + (long)n0 * MLP_W + k0, MLP_W, wave == 0 ? P + a.off.b[l] + n0 : nullptr);
+    k = j < GR_PB ? a.off.w[MLP_HIDDEN + 1] + (j - GR_PW) : a.off.b[MLP_HIDDEN + 1];
   }
+  finish_gradient(a, k, gk);
+}
+
+// An Adam step with the gradient of an earlier mlp_grad_kernel launch.
+__global__ void mlp_adam_kernel(long n, const float *__restrict__ g, AdamArgs o) {
+  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) adam_update(o, k, g[k]);
 }
 
 // Inference, all six layers in one launch: a block takes FI_R rows through the five hidden
@@ -550,49 +670,6 @@ __global__ void __launch_bounds__(256, 3) mlp_forward_fused_kernel(const bf16_t 
     y[r0 + tid] = ((s_out[0][tid] + s_out[1][tid]) + (s_out[2][tid] + s_out[3][tid])) + p[off.b[MLP_HIDDEN + 1]];
 }
 
-// the BF16 copies of parameter k (see WeightCopies)
-__device__ __forceinline__ void store_weight(const WeightCopies &wc, long k, float v, bf16_t *__restrict__ pws) {
-  const bf16_t b = to_bf16(v);
-#pragma unroll
-  for (int l = 1; l <= MLP_HIDDEN; l++) {
-    const int Kl = l == 1 ? MLP_K0 : MLP_W;
-    const long d = k - wc.w_off[l];
-    if (d >= 0 && d < (long)MLP_W * Kl) {
-      const int n = (int)(d / Kl), kk = (int)(d % Kl);
-      pws[wc.fs[l] + swz(n, kk, Kl / 16)] = b;
-      if (l >= 2) pws[wc.ts[l] + swz(kk, n, MLP_W / 16)] = b;
-    }
-  }
-}
-
-__global__ void refresh_weights_kernel(long n, const float *__restrict__ p, WeightCopies wc,
-                                       bf16_t *__restrict__ pws) {
-  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) store_weight(wc, k, p[k], pws);
-}
-
-// g = sum of the TR_SPLITS partials in range order; with update, an Adam step on p and the
-// BF16 copies refreshed.
-__global__ void mlp_adam_kernel(long n, const float *__restrict__ part, float *__restrict__ g, int update,
-                                float *__restrict__ p, float *__restrict__ mo, float *__restrict__ ve, float lr,
-                                float b1, float b2, float eps, float c1, float c2, WeightCopies wc,
-                                bf16_t *__restrict__ pws) {
-  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  float gk = 0.0f;
-#pragma unroll
-  for (int s = 0; s < TR_SPLITS; s++) gk += part[(long)s * n + k];
-  g[k] = gk;
-  if (!update) return;
-  const float m = b1 * mo[k] + (1.0f - b1) * gk;
-  const float v = b2 * ve[k] + (1.0f - b2) * gk * gk;
-  mo[k] = m;
-  ve[k] = v;
-  const float pk = p[k] - lr * (m / c1) / (sqrtf(v / c2) + eps);
-  p[k] = pk;
-  store_weight(wc, k, pk, pws);
-}
-
 __global__ void gather_rows_kernel(const bf16_t *__restrict__ X, const float *__restrict__ t, long N, int M,
                                    unsigned long long seed, bf16_t *__restrict__ Xb, float *__restrict__ tb) {
   const int m = blockIdx.x;
@@ -654,8 +731,8 @@ __device__ inline void point_features(const FeatureParams &f, double x0, double 
 
 // One thread per interior or pure-outer point (i0 in [NG, G0), i1, i2 interior) and per padding
 // row (zeros). The block's 256 rows of 128 B leave through LDS, so that a wave's store is 1 KB of
-// consecutive bytes: 272 384 rows in 18.7 us, now bound by the FP64 closed forms (64 two-byte stores per thread, 128 B apart, after
-// a clearing pass over X: 26 us and 10 us).
+// consecutive bytes: 272 384 rows in 18.7 us, now bound by the FP64 closed forms (64 two-byte
+// stores per thread, 128 B apart, after a clearing pass over X: 26 us and 10 us).
 constexpr int FEAT_C = (MLP_NFEAT + 7) / 8;  // 16-byte chunks of a row that hold features
 __global__ void __launch_bounds__(256) features_kernel(GridDims g, FeatureParams f, const double *__restrict__ xx0,
                                                        const double *__restrict__ xx1, const double *__restrict__ xx2,
@@ -717,8 +794,9 @@ __global__ void seed_state_kernel(GridDims g, long npts, const float *__restrict
 // Every thread forms the i0 averages of its 3 x 3 (i1, i2) neighbours itself: on a ghost row they
 // are those of the row's source point, because `in` holds the parity images there and the average
 // is symmetric. So the three directions are one pass over memory (5.8 us at 128x128x16, LAST 8.5;
-// as three 5.1 + 5.3 + 6.2 us and a copy back, then 7 us for v and the ghost planes). Every point writes its images: those in the
-// interior phi planes for the next pass, LAST all of them and v = eta u beside u.
+// as three 5.1 + 5.3 + 6.2 us and a copy back, then 7 us for v and the ghost planes). Every point
+// writes its images: those in the interior phi planes for the next pass, LAST all of them and
+// v = eta u beside u.
 template <bool LAST>
 __global__ void smooth_kernel(GridDims g, double eta, const double *__restrict__ in, double *__restrict__ out) {
   const int i0 = NRPYELL_NG + blockIdx.x * blockDim.x + threadIdx.x;
@@ -775,11 +853,14 @@ struct nrpyell_mlp {
   // parameter layout (FP32, concatenated): for l = 1..5: W_l [256 x K_l], b_l [256]; then w_out [256], b_out [1]
   std::vector<long> w_off, b_off, w_size;
   long n_params = 0;
+  // the network's arrays, in one allocation
+  char *params = nullptr;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
-  float *part = nullptr;  // per-range gradient partials [TR_SPLITS x n_params]
+  float *part = nullptr;  // gradient partials of layer 1 and the output layer [TR_SPLITS x GR_PART]
   bf16_t *pws = nullptr;  // BF16 W_l and W_l^T in the MFMA operand layout (WeightCopies)
   long adam_t = 0;
   int cap = 0;                       // minibatch arrays allocated for this many rows
+  bf16_t *ws = nullptr;              // ... in one allocation
   bf16_t *Ht[MLP_HIDDEN + 1] = {};   // H_l^T [width_l x M], l = 0..5
   bf16_t *dZt[MLP_HIDDEN + 1] = {};  // dZ_l^T [256 x M], l = 1..5
   float *dy = nullptr;               // per-row output gradient
@@ -795,18 +876,26 @@ struct nrpyell_mlp {
   double *seed_xx = nullptr;
   hipStream_t st = nullptr;
   ~nrpyell_mlp() {
-    (void)hipFree(p); (void)hipFree(g); (void)hipFree(m); (void)hipFree(v); (void)hipFree(part);
-    (void)hipFree(pws); (void)hipFree(loss);
+    (void)hipFree(params);
     release_seed();
     release();
     if (st) (void)hipStreamDestroy(st);
   }
   int K(int l) const { return l == 1 ? MLP_K0 : MLP_W; }
+  void alloc_params() {
+    const size_t np = (size_t)(n_params + 63) / 64 * 64, nw = (size_t)pws_size(), ng = (size_t)TR_SPLITS * GR_PART;
+    params = mlp_alloc<char>(sizeof(double) * 32 + sizeof(float) * (4 * np + ng) + sizeof(bf16_t) * nw);
+    loss = (double *)params;
+    p = (float *)(params + sizeof(double) * 32);
+    g = p + np;
+    m = g + np;
+    v = m + np;
+    pws = (bf16_t *)(v + np);
+    part = (float *)(pws + nw);
+  }
   void release() {
-    for (auto *&h : Ht) { (void)hipFree(h); h = nullptr; }
-    for (auto *&d : dZt) { (void)hipFree(d); d = nullptr; }
-    (void)hipFree(dy);
-    dy = nullptr;
+    (void)hipFree(ws);
+    ws = nullptr;
     cap = 0;
   }
   void release_seed() {
@@ -829,15 +918,18 @@ struct nrpyell_mlp {
   }
   void ensure(int M) {
     if (M <= cap) return;
-    // release first; a failed allocation below (HipFailure) leaves cap 0 and null or valid
-    // pointers only, so the next call allocates again
+    // release first; a failed allocation below (HipFailure) leaves cap 0, so the next call
+    // allocates again. mlp_grad_kernel loads whole groups of GR_D steps: up to a group past an
+    // array's end, which is in the next array or the padding behind the last one.
     release();
-    Ht[0] = mlp_alloc<bf16_t>((size_t)M * MLP_K0);
+    const size_t m0 = (size_t)M * MLP_K0, m1 = (size_t)M * MLP_W, pad = GR_D * 512;
+    ws = mlp_alloc<bf16_t>(m0 + 2 * MLP_HIDDEN * m1 + pad + 2 * (size_t)M);
+    Ht[0] = ws;
     for (int l = 1; l <= MLP_HIDDEN; l++) {
-      Ht[l] = mlp_alloc<bf16_t>((size_t)M * MLP_W);
-      dZt[l] = mlp_alloc<bf16_t>((size_t)M * MLP_W);
+      Ht[l] = ws + m0 + (l - 1) * m1;
+      dZt[l] = ws + m0 + (MLP_HIDDEN + l - 1) * m1;
     }
-    dy = mlp_alloc<float>(M);
+    dy = (float *)(ws + m0 + 2 * MLP_HIDDEN * m1 + pad);
     cap = M;
   }
   MlpOffsets offsets() const {
@@ -868,10 +960,11 @@ struct nrpyell_mlp {
     hipLaunchKernelGGL(refresh_weights_kernel, dim3((n_params + 255) / 256), dim3(256), 0, st, n_params, p, copies(),
                        pws);
   }
-  // forward, loss (added to *loss_out) and gradient partials of M minibatch rows (M a multiple
-  // of 64): rows drawn from the dataset (gather) or its first M rows
-  void loss_partials(const bf16_t *X, const float *t, long N, unsigned long long seed, int gather, int M,
-                     double *loss_out) {
+  // forward, loss (added to *loss_out) and gradient of M minibatch rows (M a multiple of 64):
+  // rows drawn from the dataset (gather) or its first M rows; with update, one Adam step at
+  // learning rate lr
+  void step(const bf16_t *X, const float *t, long N, unsigned long long seed, int gather, int M, double *loss_out,
+            int update, float lr) {
     ensure(M);
     TrainArgs a;
     a.X = X;
@@ -891,7 +984,7 @@ struct nrpyell_mlp {
     a.dy = dy;
     a.loss = loss_out;
     hipLaunchKernelGGL(mlp_train_rows_kernel, dim3(M / TR_R), dim3(64 * TR_WAVES), 0, st, a);
-    WgradArgs w;
+    GradArgs w;
     for (int l = 0; l <= MLP_HIDDEN; l++) {
       w.Ht[l] = Ht[l];
       w.dZt[l] = dZt[l];
@@ -900,26 +993,22 @@ struct nrpyell_mlp {
     w.M = M;
     w.chunk = ((M + TR_SPLITS - 1) / TR_SPLITS + 15) / 16 * 16;
     w.off = a.off;
-    w.n_params = n_params;
+    w.g = g;
+    w.update = update;
+    w.adam = update ? next_adam(lr) : AdamArgs{};
     w.part = part;
-    hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(4 * WG_GROUPS + TR_SPLITS), dim3(256), 0, st, w);
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3(GR_BLOCKS), dim3(GR_THREADS), 0, st, w);
+    hipLaunchKernelGGL(mlp_small_kernel, dim3((GR_PART + 255) / 256), dim3(256), 0, st, w);
   }
   // outputs of M feature rows (M a multiple of 64) on a stream
   void forward(const bf16_t *X, long M, float *y, hipStream_t stream) {
     hipLaunchKernelGGL(mlp_forward_fused_kernel, dim3((unsigned)((M + FI_R - 1) / FI_R)), dim3(256), 0, stream, X, pws,
                        p, offsets(), copies(), M, y);
   }
-  // g = the summed partials; with update, one Adam step at learning rate lr
-  void reduce(int update, float lr) {
-    const float b1 = 0.9f, b2 = 0.999f;
-    float c1 = 1.0f, c2 = 1.0f;
-    if (update) {
-      adam_t++;
-      c1 = 1.0f - powf(b1, (float)adam_t);
-      c2 = 1.0f - powf(b2, (float)adam_t);
-    }
-    hipLaunchKernelGGL(mlp_adam_kernel, dim3((n_params + 255) / 256), dim3(256), 0, st, n_params, part, g, update, p,
-                       m, v, lr, b1, b2, 1e-8f, c1, c2, copies(), pws);
+  // the arguments of the next Adam step (counts it)
+  AdamArgs next_adam(float lr) {
+    adam_t++;
+    return {p, m, v, pws, lr, 1.0f - powf(0.9f, (float)adam_t), 1.0f - powf(0.999f, (float)adam_t), copies()};
   }
 };
 
@@ -959,13 +1048,7 @@ extern "C" int nrpyell_mlp_create(unsigned long long seed, nrpyell_mlp **out) {
       const double a = sqrt(6.0 / fan_in) * (l == 6 ? 0.1 : 1.0);
       for (long k = 0; k < s->w_size[l]; k++) h[s->w_off[l] + k] = (float)((2 * rnd() - 1) * a);
     }
-    s->p = mlp_alloc<float>(off);
-    s->g = mlp_alloc<float>(off);
-    s->m = mlp_alloc<float>(off);
-    s->v = mlp_alloc<float>(off);
-    s->pws = mlp_alloc<bf16_t>((size_t)nrpyell_mlp::pws_size());
-    s->part = mlp_alloc<float>((size_t)TR_SPLITS * off);
-    s->loss = mlp_alloc<double>(1);
+    s->alloc_params();
     HIPCHK(hipMemcpy(s->p, h.data(), off * sizeof(float), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(s->m, 0, off * sizeof(float)));
     HIPCHK(hipMemset(s->v, 0, off * sizeof(float)));
@@ -1033,8 +1116,7 @@ extern "C" int nrpyell_mlp_loss_grad(nrpyell_mlp *s, const void *x, const float 
   return api_call([&]() -> int {
     if (check_rows(M)) return NRPYELL_EINVAL;
     HIPCHK(hipMemsetAsync(s->loss, 0, sizeof(double), s->st));
-    s->loss_partials((const bf16_t *)x, t, M, 0, 0, M, s->loss);
-    s->reduce(0, 0.0f);
+    s->step((const bf16_t *)x, t, M, 0, 0, M, s->loss, 0, 0.0f);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(loss, s->loss, sizeof(double), hipMemcpyDeviceToHost, s->st));
     if (grads_host) HIPCHK(hipMemcpyAsync(grads_host, s->g, s->n_params * sizeof(float), hipMemcpyDeviceToHost, s->st));
@@ -1046,7 +1128,7 @@ extern "C" int nrpyell_mlp_loss_grad(nrpyell_mlp *s, const void *x, const float 
 // nsteps of Adam on minibatches of `batch` rows drawn uniformly from a device dataset
 // (features BF16 [N x 64], targets FP32 [N]); cosine learning-rate decay from lr to lr/100.
 // losses (host, nsteps entries, may be null) receives each step's minibatch loss. Three
-// launches per step (rows, weight gradients, Adam); the seed of step k's draw is
+// launches per step; the seed of step k's draw is
 // seed + 0x632BE59BD9B4E019 (k + 1).
 extern "C" int nrpyell_mlp_train(nrpyell_mlp *s, const void *X, const float *t, long N, int batch, int nsteps,
                                  float lr, unsigned long long seed, double *losses) {
@@ -1056,11 +1138,10 @@ extern "C" int nrpyell_mlp_train(nrpyell_mlp *s, const void *X, const float *t, 
     double *dl = dlb.p;
     HIPCHK(hipMemsetAsync(dl, 0, (nsteps > 0 ? nsteps : 1) * sizeof(double), s->st));
     for (int k = 0; k < nsteps; k++) {
-      s->loss_partials((const bf16_t *)X, t, N, seed + 0x632BE59BD9B4E019ull * (unsigned long long)(k + 1), 1, batch,
-                       dl + k);
       const float frac = nsteps > 1 ? (float)k / (float)(nsteps - 1) : 0.0f;
       const float lrk = lr * (0.01f + 0.99f * 0.5f * (1.0f + cosf(3.14159265f * frac)));
-      s->reduce(1, lrk);
+      s->step((const bf16_t *)X, t, N, seed + 0x632BE59BD9B4E019ull * (unsigned long long)(k + 1), 1, batch, dl + k, 1,
+              lrk);
     }
     HIPCHK(hipGetLastError());
     if (losses && nsteps > 0)
@@ -1087,10 +1168,11 @@ extern "C" int nrpyell_mlp_sample_rows(const void *x_src, const float *t_src, lo
   });
 }
 
-// One Adam step with the gradient of the last nrpyell_mlp_loss_grad call (its partials).
+// One Adam step with the gradient of the last nrpyell_mlp_loss_grad call.
 extern "C" int nrpyell_mlp_adam_step(nrpyell_mlp *s, float lr) {
   return api_call([&]() -> int {
-    s->reduce(1, lr);
+    hipLaunchKernelGGL(mlp_adam_kernel, dim3((s->n_params + 255) / 256), dim3(256), 0, s->st, s->n_params, s->g,
+                       s->next_adam(lr));
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->st));
     return NRPYELL_OK;
