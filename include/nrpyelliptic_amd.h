@@ -267,8 +267,9 @@ typedef struct {
   double integration_radius;  /* L2 mask radius, 100 in the reference driver (main.c:150) */
   int tile_i0;            /* i0 width of the fused substep kernel's 256-thread tile: 16, 32
                              or 64 (0 = default); the i1 height is 256 / tile_i0            */
-  int planes;             /* i2 planes per thread: 1, or 2 with tile_i0 32/64 (0 = 2 where
-                             the tile allows it, else 1)                                    */
+  int planes;             /* i2 planes per thread: 1, or 2 with tile_i0 32/64 (0 = 1 where the
+                             tile allows no 2, or the grid is so small that one-plane blocks
+                             get a CU each; else 2)                                         */
   int outer_bc;           /* NRPYELL_OUTER_BC_RADIATION: apply_bcs_outerradiation_and_inner;
                              NRPYELL_OUTER_BC_SOMMERFELD6: the Einstein Toolkit thorn's BC
                              (nrpyell_apply_bcs_sommerfeld with f_infinity 0, falloff 3)      */
@@ -285,10 +286,9 @@ typedef struct {
                              max_iterations) decide, the stop needs log10 L2 < log10_target,
                              and the solve ends after step max_steps+1 if none passes (status
                              NRPYELL_STATUS_MAX_STEPS). FP64 single-configuration solves only. */
-  int substeps_per_launch;  /* FP64 steps of the resident solver: 2 = two RK4 substeps per
-                             launch (two launches per step; radiation outer BC, Nxx2 >= 6); 1 =
-                             one per launch; 0 = 2 where the grid and BC allow it, else 1. Both
-                             give the same states bit for bit.                               */
+  int substeps_per_launch;  /* 0 = two RK4 substeps per launch (two launches per step); 1 = one
+                             per launch; 2 = two, refused unless the outer BC is the radiation
+                             one and Nxx2 >= 6. All give the same states bit for bit.         */
 } nrpyell_solve_options;
 #define NRPYELL_STOP_EVERY_STEP 0
 #define NRPYELL_STOP_ET_THORN 1

@@ -987,12 +987,17 @@ static void plan_block_order(int ncu, int nb, int ntile0, int ntile1, int ng, Bl
   order.n = n;
 }
 
-static void pair_block_order(nrpyell_solver *s) {
-  s->order = BlockOrder{};
-  if (!s->pair_path) return;
+static int cu_count() {
   int dev = 0, ncu = 0;
   HIPCHK(hipGetDevice(&dev));
   HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  return ncu;
+}
+
+static void pair_block_order(nrpyell_solver *s) {
+  s->order = BlockOrder{};
+  if (!s->pair_path) return;
+  const int ncu = cu_count();
   const int nbc_rows = (s->g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS;
   plan_block_order(ncu, nbc_rows * s->g.N2, s->ntile0, s->ntile1, s->g.N2 / s->pl, s->order);
 }
@@ -1099,7 +1104,18 @@ extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell
       set_last_error("tile_i0 must be 16, 32 or 64");
       return NRPYELL_EINVAL;
     }
-    const int pl = s->opt.planes > 0 ? s->opt.planes : (tx >= 32 ? 2 : 1);
+    const int ty = NRPYELL_BLOCK / tx;
+    s->ntile0 = (g.N0 + tx - 1) / tx;
+    s->ntile1 = (g.N1 + ty - 1) / ty;
+    int pl = s->opt.planes;
+    if (pl <= 0) {
+      // Two planes per thread share the coefficients and most of the phi window; one plane leaves half
+      // the work per block, which is faster while those blocks still get a CU each (us per RK4 step,
+      // one / two planes: 16x16x6 13.7 / 14.6, 64x64x4 13.3 / 13.6, 64x64x8 14.1 / 14.2; past that
+      // 64x64x16 16.8 / 15.1, 96x96x8 16.9 / 15.2, 128x128x16 23.5 / 20.2).
+      const long blocks = (long)g.N2 * (s->ntile0 * s->ntile1 + (g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS);
+      pl = tx >= 32 && blocks > cu_count() ? 2 : 1;
+    }
     if (pl != 1 && !(pl == 2 && tx >= 32)) {
       set_last_error("planes must be 1, or 2 with tile_i0 32 or 64");
       return NRPYELL_EINVAL;
@@ -1107,8 +1123,9 @@ extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell
     s->tx = tx;
     s->pl = pl;
     {
-      // two substeps per launch: FP64 steps with the radiation BC; the BC blocks' reflected rows
-      // and the phi windows need Nxx1 >= 10 (checked above) and Nxx2 >= 6
+      // two substeps per launch unless the caller asks for one: the BC blocks' reflected rows need
+      // Nxx1 >= 10 (checked above), the phi windows work for any even Nxx2. Asking for two by number
+      // keeps the refusals it had when only the radiation BC and Nxx2 >= 6 had that path.
       const bool can = s->opt.outer_bc == NRPYELL_OUTER_BC_RADIATION && g.N2 >= 6;
       const int want = s->opt.substeps_per_launch;
       if (want != 0 && want != 1 && want != 2) {
@@ -1119,11 +1136,8 @@ extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell
         set_last_error("two substeps per launch need the radiation outer BC and Nxx2 >= 6");
         return NRPYELL_EINVAL;
       }
-      s->pair_path = want == 2 || (want == 0 && can);
+      s->pair_path = want != 1;
     }
-    const int ty = NRPYELL_BLOCK / tx;
-    s->ntile0 = (g.N0 + tx - 1) / tx;
-    s->ntile1 = (g.N1 + ty - 1) / ty;
     {
       // the kernels split block indices with div_by: exact while index x divisor <= 2^32
       // (the two-substep kernel's BC blocks cover fewer rows: NRPYELL_PAIR_BC_ROWS >= 8)
@@ -1650,6 +1664,7 @@ struct nrpyell_batch {
   hipStream_t stream = nullptr;
   struct Group {
     int tx = 32, pl = 1;
+    bool any_n2 = false;  // a member has fewer than 6 phi planes
     std::vector<int> members;
     SubstepArgs<double> *d_args[5] = {};   // one substep per launch: per stage 1..4
     SubstepArgs<double> *d_pair[4] = {};   // two per launch: [2 j + l], l = 0 (stages 1+2), 1 (3+4), y in ycur(j)
@@ -1686,8 +1701,9 @@ struct nrpyell_batch {
   void group_step(const Group &g, int k, hipStream_t st) const {
     if (pair) {
       const int j = k & 1;
-      launch_substep_pair_batched(g.d_pair[2 * j], g.d_block_cfg, g.d_block_first, g.nblocks, g.tx, g.pl, 1, st);
-      launch_substep_pair_batched(g.d_pair[2 * j + 1], g.d_block_cfg, g.d_block_first, g.nblocks, g.tx, g.pl, 3, st);
+      for (int l = 0; l < 2; l++)
+        launch_substep_pair_batched(g.d_pair[2 * j + l], g.d_block_cfg, g.d_block_first, g.nblocks, g.tx, g.pl,
+                                    opt.outer_bc, g.any_n2, 1 + 2 * l, st);
       return;
     }
     for (int stage = 1; stage <= 4; stage++)
@@ -1779,6 +1795,8 @@ extern "C" int nrpyell_batch_create(griddata_struct **gds, const double *dts, co
       nrpyell_solve_options o = b->opt;
       o.tile_i0 = tile_i0 ? tile_i0[k] : b->opt.tile_i0;
       o.planes = planes ? planes[k] : b->opt.planes;
+      // the other configurations fill the GPU: no one-plane blocks for a small one's sake
+      if (o.planes <= 0) o.planes = o.tile_i0 == 16 ? 1 : 2;
       nrpyell_solver *s = nullptr;
       const int rc = nrpyell_solver_create(gds[k], dts[k], &o, &s);
       if (rc != NRPYELL_OK) return rc;
@@ -1794,6 +1812,7 @@ extern "C" int nrpyell_batch_create(griddata_struct **gds, const double *dts, co
       g.tx = kv.first.first;
       g.pl = kv.first.second;
       g.members = kv.second;
+      for (int k : g.members) g.any_n2 = g.any_n2 || b->solvers[k]->g.N2 < 6;
       const int m = (int)g.members.size();
       for (int stage = 1; stage <= 4; stage++) {
         std::vector<SubstepArgs<double>> args(m);

@@ -198,9 +198,11 @@ struct BlockOrder {
 };
 template <typename T>
 void launch_substep_pair(const SubstepArgs<T> &a, int first_stage, hipStream_t st, const BlockOrder *ord = nullptr);
-// the same for many configurations in one launch (block maps as launch_substep_batched)
+// the same for many configurations in one launch (block maps as launch_substep_batched); any_n2: one
+// of them has fewer than 6 phi planes
 void launch_substep_pair_batched(const SubstepArgs<double> *cfgs, const int *block_cfg, const int *block_first,
-                                 int nblocks, int tx, int pl, int first_stage, hipStream_t st);
+                                 int nblocks, int tx, int pl, int bc_kind, bool any_n2, int first_stage,
+                                 hipStream_t st);
 template <typename T>
 void launch_substep_batched(const SubstepArgs<T> *cfgs, const int *block_cfg, const int *block_first, int nblocks,
                             int tx, int pl, int stage, hipStream_t st);

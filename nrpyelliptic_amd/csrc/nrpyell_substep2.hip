@@ -1,6 +1,8 @@
 // nrpyell_substep2.hip -- two RK4 substeps per launch (stages 1+2, then stages 3+4): the path of
-// the resident solver with the radiation outer BC, in FP64 and in the FP32 bulk phase of the
-// mixed-precision solve (templated on the arithmetic type T).
+// the resident solver, in FP64 and in the FP32 bulk phase of the mixed-precision solve (templated
+// on the arithmetic type T), with either outer BC on any even number of phi planes. Against four
+// one-substep launches per step: 128x128x16 20.2 / 26.3 us (radiation), 20.7 / 26.7 us (Sommerfeld),
+// 64x64x4 13.3 / 15.4 us.
 //
 // RK4 on  u_t = v - eta u,  v_t = c^2 (lap u + AA^2 / (8 (psi+u)^7))  couples neighbouring points
 // only through the stencil of u: the next stage's u is pointwise,
@@ -49,25 +51,65 @@ __device__ __forceinline__ T next_input(T k, T dt, T yn) {
   return fma((T)0.5, dt * k, yn);
 }
 
-// Radiation term A = -c (d_r f + f / r) at outer layer pt (pt = 0: the last interior point) of
-// apply_bcs_outerradiation_and_inner.c:290-408, as bc_body evaluates it: f(di0, di1) is f at
-// offsets (di0, di1) from the point, d_0 the 11-point stencil shifted by -max(1, pt) toward the
-// interior, d_1 the centred one; geo = (1/r, dxx0/dr, dxx1/dr, (r_0/r)^3). fd is the block's LDS
-// copy of c_fd1_shift (load_fd_table): pt differs between lanes, and a lane-indexed read of the
-// constant table is a global-memory round trip in the middle of the block's dependency chain.
-template <typename T, class F>
-__device__ __forceinline__ T radiation_A(F &&f, int pt, const T geo[4], T c, T invdx0, T invdx1, const T *fd) {
-  const int sh = pt < 1 ? 1 : pt;
+// What a kernel is built for: the radiation BC on Nxx2 >= 6 planes, the same on any (even) number of
+// planes, the Sommerfeld BC on any number. The first is a kernel of its own because the phi index
+// of the general ones costs the 128x128x16 step 1 % (20.4 against 20.2 us).
+constexpr int PAIR_RADIATION = 0, PAIR_RADIATION_ANY = 1, PAIR_SOMMERFELD = 2;
+static int pair_mode(int bc_kind, bool any) {
+  if (bc_kind != NRPYELL_OUTER_BC_RADIATION) return PAIR_SOMMERFELD;
+  return any ? PAIR_RADIATION_ANY : PAIR_RADIATION;
+}
+
+// Outgoing term A = -c (d_r f + f / r) at outer layer pt (pt = 0: the last interior point), as bc_body
+// evaluates it: f(di0, di1) is f at offsets (di0, di1) from the point, geo = (1/r, dxx0/dr, dxx1/dr,
+// (r_0/r)^3). Radiation (apply_bcs_outerradiation_and_inner.c:290-408): d_0 the
+// 11-point stencil shifted by -max(1, pt) toward the interior, d_1 the centred one; fd is the
+// block's LDS copy of c_fd1_shift (load_fd_table): pt differs between lanes, and a lane-indexed read
+// of the constant table is a global-memory round trip in the middle of the block's dependency
+// chain. Otherwise (conformally_flat_BBH_apply_bcs_sommerfeld.h:49-105): 7-point
+// stencils, backward one-sided along xx0; along xx1 forward one-sided on the first interior row
+// (`first`), centred elsewhere. Either way the layers follow from
+// rhs_pt = A_pt + (r_0/r_pt)^3 (rhs_0 - A_0).
+template <typename T, int MODE, class F>
+__device__ __forceinline__ T outer_A(F &&f, int pt, bool first, const T geo[4], T c, T invdx0, T invdx1, const T *fd) {
   T d0 = 0, d1 = 0;
+  if (MODE != PAIR_SOMMERFELD) {
+    const int sh = pt < 1 ? 1 : pt;
 #pragma unroll
-  for (int j = 0; j < 11; j++) {
-    d0 = fma(fd[sh * 11 + j], f(j - 5 - sh, 0), d0);
-    d1 = fma((T)c_fd1_shift[0][j], f(0, j - 5), d1);
+    for (int j = 0; j < 11; j++) {
+      d0 = fma(fd[sh * 11 + j], f(j - 5 - sh, 0), d0);
+      d1 = fma((T)c_fd1_shift[0][j], f(0, j - 5), d1);
+    }
+  } else {
+    d0 = (T)(-49.0 / 20.0) * f(0, 0);
+#pragma unroll
+    for (int k = 1; k < 7; k++) d0 = fma((T)c_fd1_onesided7[k], f(-k, 0), d0);
+    d0 = -d0;
+    if (first) {
+      d1 = (T)(-49.0 / 20.0) * f(0, 0);
+#pragma unroll
+      for (int k = 1; k < 7; k++) d1 = fma((T)c_fd1_onesided7[k], f(0, k), d1);
+    } else {
+      d1 = (T)(1.0 / 60.0) * f(0, 3);
+      d1 = fma((T)(-3.0 / 20.0), f(0, 2), d1);
+      d1 = fma((T)(3.0 / 4.0), f(0, 1), d1);
+      d1 = fma((T)(-3.0 / 4.0), f(0, -1), d1);
+      d1 = fma((T)(3.0 / 20.0), f(0, -2), d1);
+      d1 = fma((T)(-1.0 / 60.0), f(0, -3), d1);
+    }
   }
   d0 *= invdx0;
   d1 *= invdx1;
   const T dr = geo[1] * d0 + geo[2] * d1;
   return -c * (dr + f(0, 0) * geo[0]);
+}
+
+// Periodic plane index of the i2 arms: up to 5 planes beyond the interior ones, which is more than
+// one period of a grid with 2 or 4 planes (a power of two, so the remainder is a mask).
+template <int MODE>
+__device__ __forceinline__ int wrap2_arm(const GridDims &g, int j) {
+  if (MODE != PAIR_RADIATION && g.N2 < 6) return ((j - NG) & (g.N2 - 1)) + NG;
+  return wrap2_near(g, j);
 }
 
 // Source row, source plane and i1 orientation of a row index that may lie beyond the grid's
@@ -106,7 +148,7 @@ constexpr int bc2_lds() {
   return 2 * NRB * NT + NR1 * (24 + 10 + 24 + 2 + 12) + TYB * (10 + 30 + 8 + 10 + 2 + 12) + NRPYELL_FD_TABLE;
 }
 
-template <typename T, int PAIR, int TX, int PL>
+template <typename T, int PAIR, int TX, int PL, int MODE>
 __device__ __forceinline__ void interior2_body(const SubstepArgs<T> &a, const int tile, const int pgroup,
                                                const unsigned bid, const unsigned nblk, T *lds, double *s_red) {
   constexpr int S0 = PAIR;
@@ -159,7 +201,7 @@ __device__ __forceinline__ void interior2_body(const SubstepArgs<T> &a, const in
     if (q == 0) {
 #pragma unroll
       for (int jj = 0; jj < NW; jj++) {
-        const unsigned pw = (unsigned)wrap2_near(g, i2a - NG + jj) * s2 + k2;
+        const unsigned pw = (unsigned)wrap2_arm<MODE>(g, i2a - NG + jj) * s2 + k2;
         wxu[jj] = ld32(a.in, pw);
         wxv[jj] = ld32(a.in, nt + pw);
         wyu[jj] = PAIR == 1 ? wxu[jj] : ld32(a.yn, pw);
@@ -222,9 +264,10 @@ __device__ __forceinline__ void interior2_body(const SubstepArgs<T> &a, const in
     if (b_on) {
       const int cl = ilast - i0s + NG, by = brow + NG;  // box column of ilast, box row
       const T *box = sx[bq];
-      const T Ap = radiation_A<T>([&](int d0, int d1) { return box[(by + d1) * BX + cl + bpt + d0]; }, bpt,
+      const bool first = i1s + brow == NG;
+      const T Ap = outer_A<T, MODE>([&](int d0, int d1) { return box[(by + d1) * BX + cl + bpt + d0]; }, bpt, first,
                                   s_geo[bpt][brow], a.cOB_u, (T)g.invdx0, (T)g.invdx1, s_fd);
-      const T A0 = radiation_A<T>([&](int d0, int d1) { return box[(by + d1) * BX + cl + d0]; }, 0,
+      const T A0 = outer_A<T, MODE>([&](int d0, int d1) { return box[(by + d1) * BX + cl + d0]; }, 0, first,
                                   s_geo[0][brow], a.cOB_u, (T)g.invdx0, (T)g.invdx1, s_fd);
       const T rhs0 = fma(-eta, box[by * BX + cl], b_xv0);
       const T rhs = fma(s_geo[bpt][brow][3], rhs0 - A0, Ap);
@@ -336,7 +379,7 @@ __device__ __forceinline__ void r1_stencil_point(int t, int ilast, int &e, int &
   }
 }
 
-template <typename T, int PAIR>
+template <typename T, int PAIR, int MODE>
 __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, const int plane, T *lds) {
   constexpr int S0 = PAIR;
   constexpr int NT = NRPYELL_BLOCK, TYB = NRPYELL_PAIR_BC_ROWS;
@@ -401,8 +444,8 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
     ld2x32(a.src, 2 * p, ipsi[it], iAAc[it]);
 #pragma unroll
     for (int k = 1; k <= 5; k++) {
-      izm[it][k] = ld32(a.in, (unsigned)wrap2_near(g, pl - k) * s2 + k2);
-      izp[it][k] = ld32(a.in, (unsigned)wrap2_near(g, pl + k) * s2 + k2);
+      izm[it][k] = ld32(a.in, (unsigned)wrap2_arm<MODE>(g, pl - k) * s2 + k2);
+      izp[it][k] = ld32(a.in, (unsigned)wrap2_arm<MODE>(g, pl + k) * s2 + k2);
     }
     iyu[it] = PAIR == 1 ? (T)0 : ld32(a.yn, p);
     iyv[it] = PAIR == 1 ? (T)0 : ld32(a.yn, nt + p);
@@ -432,7 +475,7 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
   for (int r = 0; r < NARMR; r++) {
     const int k = min(tid + NT * r, NARM - 1), tr = k / 30, j = (k / 3) % 10, f = k % 3;
     const int kk = j < 5 ? -(j + 1) : j - 4;  // plane offsets -1..-5, +1..+5
-    const unsigned pa = (unsigned)wrap2_near(g, i2 + kk) * s2 + (unsigned)min(r0 + tr, g.N1 + NG - 1) * s1s + ilast;
+    const unsigned pa = (unsigned)wrap2_arm<MODE>(g, i2 + kk) * s2 + (unsigned)min(r0 + tr, g.N1 + NG - 1) * s1s + ilast;
     larm[r] = f == 0 ? ld32(a.in, pa) : f == 1 ? ld32(a.in, nt + pa) : ld32(a.yn, pa);
   }
   const T lfd = (T)load_fd_table(tid);
@@ -504,10 +547,10 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
       vrow_source(g, vr, i2, row, pl, dir);
       const int col = ilast + pt;
       sA0[e][gf][pt] = gf == 0
-          ? radiation_A<T>([&](int d0, int d1) { return BX_U(vr + dir * d1, col + d0); }, pt, sgeo[e][pt], a.cOB_u,
-                           ix0, ix1, s_fd)
-          : radiation_A<T>([&](int d0, int d1) { return BX_V(vr + dir * d1, col + d0); }, pt, sgeo[e][pt], a.cOB_v,
-                           ix0, ix1, s_fd);
+          ? outer_A<T, MODE>([&](int d0, int d1) { return BX_U(vr + dir * d1, col + d0); }, pt, row == NG, sgeo[e][pt],
+                           a.cOB_u, ix0, ix1, s_fd)
+          : outer_A<T, MODE>([&](int d0, int d1) { return BX_V(vr + dir * d1, col + d0); }, pt, row == NG, sgeo[e][pt],
+                           a.cOB_v, ix0, ix1, s_fd);
     }
   }
   __syncthreads();
@@ -551,8 +594,8 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
     const int tr = tid / 12, gf = (tid % 12) / 6, pt = tid % 6, e = tr + NG;
     if (r0 + tr < g.N1 + NG) {
       const T(*R)[12] = gf == 0 ? ru1 : rv1;
-      sA1[tr][gf][pt] = radiation_A<T>([&](int d0, int d1) { return R[e + d1][6 + pt + d0]; }, pt, sgeo[e][pt],
-                                       gf == 0 ? a.cOB_u : a.cOB_v, ix0, ix1, s_fd);
+      sA1[tr][gf][pt] = outer_A<T, MODE>([&](int d0, int d1) { return R[e + d1][6 + pt + d0]; }, pt, r0 + tr == NG,
+                                       sgeo[e][pt], gf == 0 ? a.cOB_u : a.cOB_v, ix0, ix1, s_fd);
     }
   }
   __syncthreads();
@@ -579,7 +622,7 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
 // One configuration. Without a placement table: the nbc_rows*N2 BC blocks first, then the
 // interior blocks in XCD-aware order. With one (ord.n == gridDim.x): workgroup L is logical block
 // ord.q[L], the BC blocks being logical 0 .. nb-1.
-template <typename T, int PAIR, int TX, int PL>
+template <typename T, int PAIR, int TX, int PL, int MODE>
 __global__ void __launch_bounds__(NRPYELL_BLOCK, 3) substep2_kernel(SubstepArgs<T> a, const BlockOrder ord) {
   constexpr int NL = interior2_lds<TX, PL>() > bc2_lds() ? interior2_lds<TX, PL>() : bc2_lds();
   __shared__ T lds[NL];
@@ -590,12 +633,12 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, 3) substep2_kernel(SubstepArgs<
   const unsigned L = ordered ? v : blockIdx.x;
   if (L < nb) {
     const unsigned pln = div_by(L, a.nbc_mul);
-    bc2_body<T, PAIR>(a, (int)(L - pln * (unsigned)a.nbc_rows), (int)pln, lds);
+    bc2_body<T, PAIR, MODE>(a, (int)(L - pln * (unsigned)a.nbc_rows), (int)pln, lds);
     return;
   }
   const unsigned q = ordered ? L - nb : xcd_logical(L - nb, ni), ng = (unsigned)(a.g.N2 / PL);
   const unsigned tile = div_by(q, a.ng_mul);
-  interior2_body<T, PAIR, TX, PL>(a, (int)tile, (int)(q - tile * ng), q, ni, lds, s_red);
+  interior2_body<T, PAIR, TX, PL, MODE>(a, (int)tile, (int)(q - tile * ng), q, ni, lds, s_red);
 }
 
 // Many configurations (uneven grids) in one launch, as substep_batched_kernel does for one
@@ -603,7 +646,7 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, 3) substep2_kernel(SubstepArgs<
 // q - block_first[cfg] (its BC blocks first, then its interior blocks); a configuration that has
 // converged returns at once (its own done flag). Block 0 of a configuration's interior blocks
 // of the stages-3+4 launch reduces that configuration's residual partials.
-template <int PAIR, int TX, int PL>
+template <int PAIR, int TX, int PL, int MODE>
 __global__ void __launch_bounds__(NRPYELL_BLOCK, 3)
     substep2_batched_kernel(const SubstepArgs<double> *__restrict__ cfgs, const int *__restrict__ block_cfg,
                             const int *__restrict__ block_first) {
@@ -617,52 +660,70 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, 3)
   const unsigned local = q - block_first[c], nb = (unsigned)(a.nbc_rows * a.g.N2);
   if (local < nb) {
     const unsigned pln = div_by(local, a.nbc_mul);
-    bc2_body<double, PAIR>(a, (int)(local - pln * (unsigned)a.nbc_rows), (int)pln, lds);
+    bc2_body<double, PAIR, MODE>(a, (int)(local - pln * (unsigned)a.nbc_rows), (int)pln, lds);
     return;
   }
   const unsigned li = local - nb, ng = (unsigned)(a.g.N2 / PL);
   const unsigned tile = div_by(li, a.ng_mul);
-  interior2_body<double, PAIR, TX, PL>(a, (int)tile, (int)(li - tile * ng), li, a.ntile0 * a.ntile1 * ng, lds, s_red);
+  interior2_body<double, PAIR, TX, PL, MODE>(a, (int)tile, (int)(li - tile * ng), li, a.ntile0 * a.ntile1 * ng, lds, s_red);
 }
 
-template <int PAIR>
+template <int V>
+struct IntC {
+  static constexpr int value = V;
+};
+template <class F>
+static void by_stage_and_mode(int first_stage, int mode, F &&go) {
+  auto with = [&](auto m) {
+    if (first_stage == 1) go(IntC<1>{}, m);
+    else go(IntC<3>{}, m);
+  };
+  if (mode == PAIR_RADIATION) with(IntC<PAIR_RADIATION>{});
+  else if (mode == PAIR_RADIATION_ANY) with(IntC<PAIR_RADIATION_ANY>{});
+  else with(IntC<PAIR_SOMMERFELD>{});
+}
+
+template <int PAIR, int MODE>
 static void launch_pair_batched(const SubstepArgs<double> *cfgs, const int *block_cfg, const int *block_first,
                                 int nblocks, int tx, int pl, hipStream_t st) {
   dim3 grd(nblocks), blk(NRPYELL_BLOCK);
   if (pl == 2) {
     switch (tx) {
-      case 64: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 64, 2>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
-      default: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 32, 2>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
+      case 64: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 64, 2, MODE>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
+      default: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 32, 2, MODE>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
     }
     return;
   }
   switch (tx) {
-    case 16: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 16, 1>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
-    case 64: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 64, 1>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
-    default: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 32, 1>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
+    case 16: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 16, 1, MODE>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
+    case 64: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 64, 1, MODE>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
+    default: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 32, 1, MODE>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
   }
 }
 
 void launch_substep_pair_batched(const SubstepArgs<double> *cfgs, const int *block_cfg, const int *block_first,
-                                 int nblocks, int tx, int pl, int first_stage, hipStream_t st) {
-  if (first_stage == 1) launch_pair_batched<1>(cfgs, block_cfg, block_first, nblocks, tx, pl, st);
-  else launch_pair_batched<3>(cfgs, block_cfg, block_first, nblocks, tx, pl, st);
+                                 int nblocks, int tx, int pl, int bc_kind, bool any_n2, int first_stage,
+                                 hipStream_t st) {
+  auto go = [&](auto pair, auto mode) {
+    launch_pair_batched<decltype(pair)::value, decltype(mode)::value>(cfgs, block_cfg, block_first, nblocks, tx, pl, st);
+  };
+  by_stage_and_mode(first_stage, pair_mode(bc_kind, any_n2), go);
 }
 
-template <typename T, int PAIR>
+template <typename T, int PAIR, int MODE>
 static void launch_pair(const SubstepArgs<T> &a, hipStream_t st, const BlockOrder &o) {
   dim3 grd(a.nbc_rows * a.g.N2 + a.ntile0 * a.ntile1 * (a.g.N2 / a.pl)), blk(NRPYELL_BLOCK);
   if (a.pl == 2) {
     switch (a.tx) {
-      case 64: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 64, 2>), grd, blk, 0, st, a, o); break;
-      default: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 2>), grd, blk, 0, st, a, o); break;
+      case 64: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 64, 2, MODE>), grd, blk, 0, st, a, o); break;
+      default: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 2, MODE>), grd, blk, 0, st, a, o); break;
     }
     return;
   }
   switch (a.tx) {
-    case 16: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 16, 1>), grd, blk, 0, st, a, o); break;
-    case 64: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 64, 1>), grd, blk, 0, st, a, o); break;
-    default: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 1>), grd, blk, 0, st, a, o); break;
+    case 16: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 16, 1, MODE>), grd, blk, 0, st, a, o); break;
+    case 64: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 64, 1, MODE>), grd, blk, 0, st, a, o); break;
+    default: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 1, MODE>), grd, blk, 0, st, a, o); break;
   }
 }
 
@@ -670,8 +731,8 @@ template <typename T>
 void launch_substep_pair(const SubstepArgs<T> &a, int first_stage, hipStream_t st, const BlockOrder *ord) {
   static const BlockOrder none{};
   const BlockOrder &o = ord ? *ord : none;
-  if (first_stage == 1) launch_pair<T, 1>(a, st, o);
-  else launch_pair<T, 3>(a, st, o);
+  auto go = [&](auto pair, auto mode) { launch_pair<T, decltype(pair)::value, decltype(mode)::value>(a, st, o); };
+  by_stage_and_mode(first_stage, pair_mode(a.bc_kind, a.g.N2 < 6), go);
 }
 template void launch_substep_pair<double>(const SubstepArgs<double> &, int, hipStream_t, const BlockOrder *);
 template void launch_substep_pair<float>(const SubstepArgs<float> &, int, hipStream_t, const BlockOrder *);
