@@ -784,6 +784,7 @@ struct nrpyell_solver {
     a.state = nullptr;
     a.l2_volume = 0.0;
     a.l2_target = 0.0;
+    a.copy = nullptr;
     return a;
   }
 
@@ -869,12 +870,11 @@ struct nrpyell_solver {
     return k;
   }
   // Metric coefficients from the rfm arrays and the c^2-folded coefficient and source tables
-  // from auxevol: the only reads of those arrays. Raises `bad` (cleared first) when the wave
-  // speed varies along xx2.
-  // also_clear: another flag to zero with the wave-speed check's (the drop-in step's done flag)
-  // (the flags are zeroed by a kernel, not a memset: this runs inside the drop-in step's graph)
-  void refresh_tables(hipStream_t st, int *also_clear = nullptr) {
-    launch_tables(g, &gd->rfmstruct, gd->gridfuncs.auxevol_gfs, w2d, coef64, kc64, kc32, src64, bad, also_clear, st);
+  // from auxevol: the only reads of those arrays. Raises `bad` when the wave
+  // speed varies along xx2 (the flag is the host's own memory: whoever launches the kernels zeroes
+  // it first).
+  void refresh_tables(hipStream_t st) {
+    launch_tables(g, &gd->rfmstruct, gd->gridfuncs.auxevol_gfs, w2d, coef64, kc64, kc32, src64, bad, st);
     HIPCHK(hipGetLastError());
   }
   // The fused kernels keep only the interior phi planes current; this fills the ghost planes
@@ -1611,28 +1611,27 @@ extern "C" void MoL_step_forward_in_time(griddata_struct *griddata, const REAL d
       }
     }
     s->dt = dt;
-    // one graph per solver: table refresh (the rfm and auxevol arrays are re-read every call),
-    // the RK4 step (two launches of two substeps where the grid allows, then y back to
-    // y_n_gfs), the phi ghost planes; recaptured when dt, eta or the outer wave speeds change
+    // one graph per solver: table refresh (the rfm and auxevol arrays are re-read every call) and
+    // the RK4 step in two launches that leave the result in y_n_gfs, ghosts included; recaptured
+    // when dt, eta or the outer wave speeds change. (The solver's done flag stays 0: no launch of
+    // this graph makes a residual check.)
     const nrpyell_solver::GraphKey k = s->graph_key(false, 0.0);
     if (!s->graph_step || !s->key_step.same(k)) {
       if (s->graph_step) (void)hipGraphExecDestroy(s->graph_step);
       s->graph_step = nullptr;
       hipGraph_t gr;
       HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-      s->refresh_tables(s->stream, &s->dstate->done);
-      if (s->pair_path) {
-        s->step64_pair(s->stream, 0, false);
-        s->finish(s->stream, 1);
-      } else {
-        s->step64(s->stream);
-        s->finish(s->stream, 0);
-      }
+      s->refresh_tables(s->stream);
+      SubstepArgs<double> a = s->args<double>(1, gf.y_n_gfs, gf.k_odd_gfs, nullptr, gf.y_nplus1_running_total_gfs,
+                                              s->src64, s->kc64, s->geo64);
+      s->pair_layout(a);
+      launch_step_in_place(a, gf.y_n_gfs, gf.k_odd_gfs, gf.k_even_gfs, s->stream, &s->order);
       HIPCHK(hipStreamEndCapture(s->stream, &gr));
       HIPCHK(hipGraphInstantiate(&s->graph_step, gr, nullptr, nullptr, 0));
       HIPCHK(hipGraphDestroy(gr));
       s->key_step = k;
     }
+    *(volatile int *)s->bad_host = 0;
     HIPCHK(hipGraphLaunch(s->graph_step, s->stream));
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s->stream));

@@ -158,6 +158,7 @@ struct SubstepArgs {
   double *l2_partial;         // one partial sum per block
   SolverDeviceState *state;   // convergence state
   double l2_volume, l2_target;
+  T *copy;  // launch_step_in_place: a second copy of y, written by the first launch
 };
 
 
@@ -167,10 +168,10 @@ void launch_rhs_exact(const GridDims &g, const rfm_struct *rfm, const double *au
 void launch_residual_exact(const GridDims &g, const rfm_struct *rfm, const double *aux, const double *in,
                            double *out, hipStream_t st);
 // the solver's tables from rfm and auxevol: metric coefficients (coef64), their c^2-folded record
-// with the L2 weight (kc64, kc32), the per-point source (src); *bad raised where the wave speed
-// varies along xx2; *bad and *also_clear (when given) zeroed first, by the same launch
+// with the L2 weight (kc64, kc32), the per-point source on the interior phi planes (src); *bad, which
+// the caller zeroes first, raised where the wave speed varies along xx2
 void launch_tables(const GridDims &g, const rfm_struct *rfm, const double *aux, const double *w2d, double *coef64,
-                   double *kc64, float *kc32, double *src, int *bad, int *also_clear, hipStream_t st);
+                   double *kc64, float *kc32, double *src, int *bad, hipStream_t st);
 template <typename T>
 void launch_fill_ghost_planes(const GridDims &g, T *y, int ngf, hipStream_t st);
 // dst = src with dst's ghost phi planes filled from their sources (copy + fill_ghost_planes)
@@ -198,7 +199,12 @@ struct BlockOrder {
 };
 template <typename T>
 void launch_substep_pair(const SubstepArgs<T> &a, int first_stage, hipStream_t st, const BlockOrder *ord = nullptr);
-// the same for many configurations in one launch (block maps as launch_substep_batched); any_n2: one
+// One RK4 step of two launches whose result lands in y_n_gfs itself, ghosts included (the drop-in
+// step): the first launch also copies y to `copy`, the second reads y there and writes y_n with all
+// its parity images, so no pass over the state follows. FP64, radiation BC, 32-wide tiles.
+void launch_step_in_place(SubstepArgs<double> a, double *y_n, double *k_odd, double *copy, hipStream_t st,
+                          const BlockOrder *ord);
+// launch_substep_pair for many configurations in one launch (block maps as launch_substep_batched); any_n2: one
 // of them has fewer than 6 phi planes
 void launch_substep_pair_batched(const SubstepArgs<double> *cfgs, const int *block_cfg, const int *block_first,
                                  int nblocks, int tx, int pl, int bc_kind, bool any_n2, int first_stage,

@@ -2,9 +2,9 @@
 // RK4 substeps (nrpyell_substep.hip, nrpyell_substep2.hip). One thread per grid point or list
 // entry, i0 across lanes so that loads coalesce:
 //   rhs_exact_kernel, residual_exact_kernel   rhs_eval.c:7-117, residual_all_points.c:7-112 with
-//                           the reference FMA tree (drop-in entry points; 64 x 4 tiles, x0/x1
-//                           stencil arms staged in LDS)
-//   coef_fold_kernel, fold_source_kernel      the solver's tables from rfm and auxevol
+//                           the reference FMA tree (drop-in entry points; 32 x 8 tiles of two planes,
+//                           x0/x1 stencil arms staged in LDS)
+//   tables_kernel           the solver's tables from rfm and auxevol
 //   residual_l2_partial_kernel, l2_partial_kernel, l2_finalize_kernel   residual + masked,
 //                           volume-weighted sum of squares, partials reduced in a fixed order
 //                           (L2_norm_of_gf.c:6-43)
@@ -19,6 +19,7 @@
 
 #include "nrpyell_common.h"
 #include "nrpyell_internal.h"
+#include "nrpyell_stencil.h"
 
 #define NG NRPYELL_NG
 
@@ -40,126 +41,186 @@ __device__ inline double fd2_exact(const double m[6], const double p[6], double 
                  fma(1.0 / 3150.0, m[5] + p[5], -fma(5.0 / 1008.0, m[4] + p[4], fma(5.0 / 21.0, m[2] + p[2], c0)))));
 }
 
+// The factors of the reference's expression that depend on (i0, i1) only.
+struct ExactCoef {
+  double a0, a2, B0, a0f1p, f1, K22;
+};
+
+__device__ __forceinline__ ExactCoef exact_coef(const double f0, const double f0p, const double f0pp, const double f1,
+                                                const double f1p, const double f2, const double f2_0, const double f3,
+                                                const double f3p) {
+  ExactCoef k;
+  k.a0 = 1.0 / (f2 * f2);
+  k.a2 = (f3 * f3) / (f0p * f0p);
+  const double a3 = 1.0 / ((f2 * f2) * f2);
+  const double num = fma(f3, fma(f0p, f2_0, f0pp * f2), -(f0p * (f2 * f3p)));
+  const double tA = num / ((f0p * f0p) * f0p);
+  const double tB = ((k.a0 * -1.0) * ((f3 * f3) / f0p)) / f0;
+  const double inner = fma(k.a2, a3 * f2_0, -tB);
+  k.B0 = fma(a3 * f3, tA, -inner);
+  k.a0f1p = k.a0 * f1p;
+  k.f1 = f1;
+  k.K22 = (1.0 / (f1 * f1)) / (f0 * f0);
+  return k;
+}
+
 // Flat-space Laplacian in SinhSymTP plus AA^2/(8 (psi+u)^7), reference expression tree, from the
 // stencil arms m*/p* (u at offsets -k / +k along x0, x1, x2) and the centre value uu.
-__device__ inline double lap_source_exact(const GridDims &g, const RfmPtrs &r, const double m0[6], const double p0[6],
-                                          const double m1[6], const double p1[6], const double m2[6],
-                                          const double p2[6], double uu, int i0, int i1, double psi, double AA) {
+__device__ __forceinline__ double lap_source_exact(const GridDims &g, const ExactCoef &k, const double m0[6],
+                                                   const double p0[6], const double m1[6], const double p1[6],
+                                                   const double m2[6], const double p2[6], double uu, double psi,
+                                                   double AA) {
   const double c0 = (5269.0 / 1800.0) * uu;
   const double dD0 = g.invdx0 * fd1_exact(m0, p0);
   const double dD1 = g.invdx1 * fd1_exact(m1, p1);
   const double dDD00 = (g.invdx0 * g.invdx0) * fd2_exact(m0, p0, c0);
   const double dDD11 = (g.invdx1 * g.invdx1) * fd2_exact(m1, p1, c0);
   const double dDD22 = (g.invdx2 * g.invdx2) * fd2_exact(m2, p2, c0);
-  const long k2 = i0 + (long)g.G0 * i1;
-  const double f0 = r.f0[i0], f0p = r.f0_D0[i0], f0pp = r.f0_DD00[i0];
-  const double f1 = r.f1[i1], f1p = r.f1_D1[i1];
-  const double f2 = r.f2[k2], f2_0 = r.f2_D0[k2];
-  const double f3 = r.f3[i0], f3p = r.f3_D0[i0];
-  const double a0 = 1.0 / (f2 * f2);
-  const double a2 = (f3 * f3) / (f0p * f0p);
-  const double a3 = 1.0 / ((f2 * f2) * f2);
   const double X = psi + uu;
   const double X7 = (((((X * X) * X) * X) * X) * X) * X;
-  const double num = fma(f3, fma(f0p, f2_0, f0pp * f2), -(f0p * (f2 * f3p)));
-  const double tA = num / ((f0p * f0p) * f0p);
-  const double tB = ((a0 * -1.0) * ((f3 * f3) / f0p)) / f0;
-  const double inner = fma(a2, a3 * f2_0, -tB);
-  const double B0 = fma(a3 * f3, tA, -inner);
-  double e = fma(a0, dDD11, -(dD0 * B0));
-  e = fma(a0 * f1p, dD1 / f1, e);
+  double e = fma(k.a0, dDD11, -(dD0 * k.B0));
+  e = fma(k.a0f1p, dD1 / k.f1, e);
   e = fma(1.0 / 8.0, AA / X7, e);
-  e = fma(a0, a2 * dDD00, e);
-  e = fma(dDD22, (1.0 / (f1 * f1)) / (f0 * f0), e);
+  e = fma(k.a0, k.a2 * dDD00, e);
+  e = fma(dDD22, k.K22, e);
   return e;
 }
 
-// The drop-in kernels work on 64 x 4 tiles of one plane: the tile's u with its 5-point halos in
-// x0 and x1 is staged in LDS (the x0 and x1 arms of every point are read from there), the x2
-// arms come from global memory. Only where the values come from differs from a per-point
-// gather: each point's arithmetic is the reference's expression tree.
-#define EX_TX 64
-#define EX_TY 4
+// The drop-in kernels work on 32 x 8 tiles of P consecutive planes, one (i0,i1) column of P
+// points per thread: eight of the expression's ten divisions depend on (i0,i1) only and are done
+// once, and the x2 arms share one window of planes. The tile's u with its 5-point halos in x0 and x1
+// is staged in LDS; every global load is issued before the barrier, from clamped indices (a clamped
+// value is never used by a point of the grid), so a block waits for memory once. Blocks are in
+// XCD-aware order, plane group fastest, so that an XCD's L2 serves the arms and halos. Each point's
+// arithmetic is the reference's expression tree, so the values are bit-exact. Against 64 x 4 tiles
+// of one plane that waited for the halo before they loaded the rest: residual at 128x128x16 6.6 / 8.2
+// us, RHS at 200x130x16 10.3 / 15.2 us.
+#define EX_TX 32
+#define EX_TY 8
 #define EX_BX (EX_TX + 2 * NG)
 #define EX_BY (EX_TY + 2 * NG)
-
-struct ExactTile {
-  int i0, i1, i2;
-  long p;
-  bool valid;
+struct ExactGrid {
+  unsigned n, nt0, nz;                    // blocks, tiles along x0, plane groups
+  unsigned long long nz_mul, nt0_mul;     // div_mul of nz and nt0, 0 where that would not be exact
 };
 
-// Stage the tile's box (rows i1s-5 .. i1s+8, columns i0s-5 .. i0s+68, clamped to the grid: a
-// clamped value is never read by a point of the grid) and wait for the whole block.
-__device__ __forceinline__ ExactTile exact_tile(const GridDims &g, const double *u, double *box) {
-  const int i0s = NG + blockIdx.x * EX_TX, i1s = NG + blockIdx.y * EX_TY, i2 = NG + blockIdx.z;
-  const long base = (long)i2 * g.G0 * g.G1;
-  for (int k = threadIdx.y * EX_TX + threadIdx.x; k < EX_BX * EX_BY; k += EX_TX * EX_TY) {
-    const int bx = k % EX_BX, by = k / EX_BX;
-    const int j0 = min(i0s - NG + bx, g.G0 - 1), j1 = min(i1s - NG + by, g.G1 - 1);
-    box[k] = u[base + (long)j1 * g.G0 + j0];
-  }
-  __syncthreads();
-  ExactTile t;
-  t.i0 = i0s + (int)threadIdx.x;
-  t.i1 = i1s + (int)threadIdx.y;
-  t.i2 = i2;
-  t.p = idx3(g, t.i0, t.i1, i2);
-  t.valid = t.i0 < g.N0 + NG && t.i1 < g.N1 + NG;
-  return t;
+__device__ __forceinline__ unsigned exact_div(unsigned q, unsigned d, unsigned long long mul) {
+  return mul ? div_by(q, mul) : q / d;
 }
 
-__device__ __forceinline__ double exact_point(const GridDims &g, const RfmPtrs &r, const double *u, const double *box,
-                                              const ExactTile &t, double psi, double AA) {
-  double m0[6], p0[6], m1[6], p1[6], m2[6], p2[6];
-  const int c = ((int)threadIdx.y + NG) * EX_BX + (int)threadIdx.x + NG;
-  const long s2 = (long)g.G0 * g.G1;
+// RHS: out = (v - eta u | c^2 e) with e the expression's value; otherwise out = e.
+template <bool RHS, int P>
+__device__ __forceinline__ void exact_column(const GridDims &g, const RfmPtrs &r, const double *__restrict__ aux,
+                                             const double *__restrict__ u, double *__restrict__ out, double eta,
+                                             const ExactGrid &x) {
+  constexpr int NT = EX_TX * EX_TY, BOX = EX_BX * EX_BY, NR = (BOX + NT - 1) / NT, NW = P + 2 * NG;
+  __shared__ double box[P][NR * NT];
+  const unsigned b = xcd_logical(blockIdx.x, x.n), tile = exact_div(b, x.nz, x.nz_mul),
+                 t1 = exact_div(tile, x.nt0, x.nt0_mul);
+  const int i2a = NG + P * (int)(b - tile * x.nz), i0s = NG + EX_TX * (int)(tile - t1 * x.nt0),
+            i1s = NG + EX_TY * (int)t1;
+  const int tid = threadIdx.x, tx = tid % EX_TX, ty = tid / EX_TX, i0 = i0s + tx, i1 = i1s + ty;
+  const int i0c = min(i0, g.G0 - 1), i1c = min(i1, g.G1 - 1);
+  const long s2 = (long)g.G0 * g.G1, k2 = i0c + (long)g.G0 * i1c, nt = g.ntot;
+  double bx[P][NR], w[NW], psi[P], AA[P], v[P], c[P];
 #pragma unroll
-  for (int k = 1; k <= 5; k++) {
-    m0[k] = box[c - k]; p0[k] = box[c + k];
-    m1[k] = box[c - k * EX_BX]; p1[k] = box[c + k * EX_BX];
-    m2[k] = u[t.p - k * s2]; p2[k] = u[t.p + k * s2];
+  for (int q = 0; q < P; q++) {
+    const double *pl = u + min(i2a + q, g.G2 - 1) * s2;
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      const int e = tid + NT * k, j0 = min(i0s - NG + e % EX_BX, g.G0 - 1), j1 = min(i1s - NG + e / EX_BX, g.G1 - 1);
+      bx[q][k] = pl[(long)j1 * g.G0 + j0];
+    }
   }
-  return lap_source_exact(g, r, m0, p0, m1, p1, m2, p2, box[c], t.i0, t.i1, psi, AA);
+#pragma unroll
+  for (int j = 0; j < NW; j++) w[j] = u[min(i2a - NG + j, g.G2 - 1) * s2 + k2];
+#pragma unroll
+  for (int q = 0; q < P; q++) {
+    const long p = min(i2a + q, g.G2 - 1) * s2 + k2;
+    psi[q] = aux[PSI_BACKGROUNDGF * nt + p];
+    AA[q] = aux[ADD_TIMES_AUUGF * nt + p];
+    if (RHS) {
+      v[q] = u[nt + p];
+      c[q] = aux[WAVESPEEDGF * nt + p];
+    }
+  }
+  const double f0 = r.f0[i0c], f0p = r.f0_D0[i0c], f0pp = r.f0_DD00[i0c], f1 = r.f1[i1c], f1p = r.f1_D1[i1c],
+               f2 = r.f2[k2], f2_0 = r.f2_D0[k2], f3 = r.f3[i0c], f3p = r.f3_D0[i0c];
+#pragma unroll
+  for (int q = 0; q < P; q++)
+#pragma unroll
+    for (int k = 0; k < NR; k++) box[q][tid + NT * k] = bx[q][k];
+  const ExactCoef K = exact_coef(f0, f0p, f0pp, f1, f1p, f2, f2_0, f3, f3p);
+  __syncthreads();
+  if (i0 >= g.N0 + NG || i1 >= g.N1 + NG) return;
+  const int cb = (ty + NG) * EX_BX + tx + NG;
+#pragma unroll
+  for (int q = 0; q < P; q++) {
+    if (i2a + q >= g.N2 + NG) break;  // odd plane count
+    double m0[6], p0[6], m1[6], p1[6], m2[6], p2[6];
+#pragma unroll
+    for (int k = 1; k <= 5; k++) {
+      m0[k] = box[q][cb - k]; p0[k] = box[q][cb + k];
+      m1[k] = box[q][cb - k * EX_BX]; p1[k] = box[q][cb + k * EX_BX];
+      m2[k] = w[NG + q - k]; p2[k] = w[NG + q + k];
+    }
+    const long p = (i2a + q) * s2 + k2;
+    const double e = lap_source_exact(g, K, m0, p0, m1, p1, m2, p2, w[NG + q], psi[q], AA[q]);
+    out[p] = RHS ? fma(-eta, w[NG + q], v[q]) : e;
+    if (RHS) out[nt + p] = (c[q] * c[q]) * e;
+  }
 }
 
-__global__ void __launch_bounds__(256) rhs_exact_kernel(GridDims g, RfmPtrs r, const double *aux, const double *in,
-                                                        double *out, double eta) {
-  __shared__ double box[EX_BX * EX_BY];
-  const ExactTile t = exact_tile(g, in, box);
-  if (!t.valid) return;
-  const long p = t.p, nt = g.ntot;
-  const double *u = in, *v = in + nt;
-  const double e = exact_point(g, r, u, box, t, aux[PSI_BACKGROUNDGF * nt + p], aux[ADD_TIMES_AUUGF * nt + p]);
-  const double c = aux[WAVESPEEDGF * nt + p];
-  out[p] = fma(-eta, u[p], v[p]);
-  out[nt + p] = (c * c) * e;
+template <int P>
+__global__ void __launch_bounds__(EX_TX *EX_TY) rhs_exact_kernel(GridDims g, RfmPtrs r, const double *aux,
+                                                                 const double *in, double *out, double eta,
+                                                                 ExactGrid x) {
+  exact_column<true, P>(g, r, aux, in, out, eta, x);
 }
 
-__global__ void __launch_bounds__(256) residual_exact_kernel(GridDims g, RfmPtrs r, const double *aux,
-                                                             const double *in, double *out) {
-  __shared__ double box[EX_BX * EX_BY];
-  const ExactTile t = exact_tile(g, in, box);
-  if (!t.valid) return;
-  const long p = t.p, nt = g.ntot;
-  out[p] = exact_point(g, r, in, box, t, aux[PSI_BACKGROUNDGF * nt + p], aux[ADD_TIMES_AUUGF * nt + p]);
+template <int P>
+__global__ void __launch_bounds__(EX_TX *EX_TY) residual_exact_kernel(GridDims g, RfmPtrs r, const double *aux,
+                                                                      const double *in, double *out, ExactGrid x) {
+  exact_column<false, P>(g, r, aux, in, out, 0.0, x);
+}
+
+// Two planes per thread where one would give more blocks than the GPU has CUs (256): below that a
+// block per plane is the shorter chain (16x16x6: 14.6 us per rhs_eval call against 14.9 with two).
+static ExactGrid exact_grid(const GridDims &g, int &planes) {
+  ExactGrid x;
+  x.nt0 = (g.N0 + EX_TX - 1) / EX_TX;
+  const unsigned tiles = x.nt0 * ((g.N1 + EX_TY - 1) / EX_TY);
+  planes = (long)tiles * g.N2 <= 256 ? 1 : 2;
+  x.nz = (g.N2 + planes - 1) / planes;
+  x.n = tiles * x.nz;
+  // the multiply-high quotients are exact while index x divisor <= 2^32
+  x.nz_mul = (double)x.n * x.nz <= 4294967296.0 ? div_mul(x.nz) : 0;
+  x.nt0_mul = (double)tiles * x.nt0 <= 4294967296.0 ? div_mul(x.nt0) : 0;
+  return x;
+}
+
+static RfmPtrs exact_rfm(const rfm_struct *rfm) {
+  return {rfm->f0_of_xx0, rfm->f0_of_xx0__D0, rfm->f0_of_xx0__DD00, rfm->f1_of_xx1, rfm->f1_of_xx1__D1,
+          rfm->f2_of_xx0_xx1, rfm->f2_of_xx0_xx1__D0, rfm->f3_of_xx0, rfm->f3_of_xx0__D0};
 }
 
 void launch_rhs_exact(const GridDims &g, const rfm_struct *rfm, const double *aux, const double *in, double *out,
                       double eta, hipStream_t st) {
-  RfmPtrs r{rfm->f0_of_xx0, rfm->f0_of_xx0__D0, rfm->f0_of_xx0__DD00, rfm->f1_of_xx1, rfm->f1_of_xx1__D1,
-            rfm->f2_of_xx0_xx1, rfm->f2_of_xx0_xx1__D0, rfm->f3_of_xx0, rfm->f3_of_xx0__D0};
-  dim3 blk(EX_TX, EX_TY), grd((g.N0 + EX_TX - 1) / EX_TX, (g.N1 + EX_TY - 1) / EX_TY, g.N2);
-  if (out)
-    hipLaunchKernelGGL(rhs_exact_kernel, grd, blk, 0, st, g, r, aux, in, out, eta);
+  if (!out) return;
+  int planes;
+  const ExactGrid x = exact_grid(g, planes);
+  const dim3 grd(x.n), blk(EX_TX * EX_TY);
+  if (planes == 1) hipLaunchKernelGGL(rhs_exact_kernel<1>, grd, blk, 0, st, g, exact_rfm(rfm), aux, in, out, eta, x);
+  else hipLaunchKernelGGL(rhs_exact_kernel<2>, grd, blk, 0, st, g, exact_rfm(rfm), aux, in, out, eta, x);
 }
 
 void launch_residual_exact(const GridDims &g, const rfm_struct *rfm, const double *aux, const double *in,
                            double *out, hipStream_t st) {
-  RfmPtrs r{rfm->f0_of_xx0, rfm->f0_of_xx0__D0, rfm->f0_of_xx0__DD00, rfm->f1_of_xx1, rfm->f1_of_xx1__D1,
-            rfm->f2_of_xx0_xx1, rfm->f2_of_xx0_xx1__D0, rfm->f3_of_xx0, rfm->f3_of_xx0__D0};
-  dim3 blk(EX_TX, EX_TY), grd((g.N0 + EX_TX - 1) / EX_TX, (g.N1 + EX_TY - 1) / EX_TY, g.N2);
-  hipLaunchKernelGGL(residual_exact_kernel, grd, blk, 0, st, g, r, aux, in, out);
+  int planes;
+  const ExactGrid x = exact_grid(g, planes);
+  const dim3 grd(x.n), blk(EX_TX * EX_TY);
+  if (planes == 1) hipLaunchKernelGGL(residual_exact_kernel<1>, grd, blk, 0, st, g, exact_rfm(rfm), aux, in, out, x);
+  else hipLaunchKernelGGL(residual_exact_kernel<2>, grd, blk, 0, st, g, exact_rfm(rfm), aux, in, out, x);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -174,64 +235,65 @@ void launch_residual_exact(const GridDims &g, const rfm_struct *rfm, const doubl
 //   B   = f3 (f3 (f0' d0f2 + f0'' f2) - f0' f2 f3')/(f0'^3 f2^3) - d0f2 f3^2/(f0'^2 f2^3)
 //         - f3^2/(f0 f0' f2^2)
 // ---------------------------------------------------------------------------------------
-// coef_fold_kernel writes K00 .. K0 (coef, read by the residual check) and the same five times
-// c^2 plus the L2 weight / c^4 (kc64, kc32: the fused kernels' per-(i0,i1) record, c the wave
-// speed on the plane i2 = NG), and zeroes the flags it is given (thread 0 of block (0, 0)):
-// the wave-speed check's, which fold_source_kernel then raises, and the caller's.
-__global__ void coef_fold_kernel(GridDims g, RfmPtrs r, const double *aux, const double *w2d, double *coef,
-                                 double *kc64, float *kc32, int *flag0, int *flag1) {
-  const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i1 = blockIdx.y;
-  if (i0 == 0 && i1 == 0) {
-    *flag0 = 0;
-    if (flag1) *flag1 = 0;
-  }
-  if (i0 >= g.G0) return;
-  const long k2 = i0 + (long)g.G0 * i1, n2 = (long)g.G0 * g.G1;
-  const double f0 = r.f0[i0], f0p = r.f0_D0[i0], f0pp = r.f0_DD00[i0];
-  const double f1 = r.f1[i1], f1p = r.f1_D1[i1];
-  const double f2 = r.f2[k2], f2_0 = r.f2_D0[k2];
-  const double f3 = r.f3[i0], f3p = r.f3_D0[i0];
-  const double a0 = 1.0 / (f2 * f2), a2 = (f3 * f3) / (f0p * f0p), a3 = a0 / f2;
-  const double B = f3 * a3 * (f3 * (f0p * f2_0 + f0pp * f2) - f0p * f2 * f3p) / (f0p * f0p * f0p) -
-                   a2 * a3 * f2_0 - a0 * (f3 * f3) / (f0p * f0);
-  const double K[5] = {a0 * a2 * (g.invdx0 * g.invdx0), a0 * (g.invdx1 * g.invdx1),
-                       (1.0 / (f1 * f1)) / (f0 * f0) * (g.invdx2 * g.invdx2), a0 * f1p / f1 * g.invdx1,
-                       -B * g.invdx0};
-  const double c = aux[WAVESPEEDGF * g.ntot + idx3(g, i0, i1, NG)], c2 = c * c;
+// tables_kernel, one launch for both tables (two launches of 4.2 and 5.3 us at 128x128x16, the first
+// a few waves of divisions that left the chip idle; together 6.3 us): blocks below ncoef write
+// K00 .. K0 (coef, read by the residual check) and the same five times c^2 plus the L2 weight / c^4
+// (kc64, kc32: the fused kernels' per-(i0,i1) record, c the wave speed on the plane i2 = NG); the
+// other blocks write (psi, c^2 AA^2 / 8) interleaved per point of the interior planes (one 16-byte
+// load in the fused kernels) and raise *bad where the wave speed at an interior point differs from
+// its value on the plane i2 = NG.
+__global__ void __launch_bounds__(256) tables_kernel(GridDims g, RfmPtrs r, const double *__restrict__ aux,
+                                                     const double *__restrict__ w2d, double *__restrict__ coef,
+                                                     double *__restrict__ kc64, float *__restrict__ kc32,
+                                                     double *__restrict__ src, int *bad, unsigned ncoef) {
+  const unsigned plane = (unsigned)(g.G0 * g.G1);
+  const long nt = g.ntot;
+  if (blockIdx.x < ncoef) {
+    const unsigned k2 = blockIdx.x * 256 + threadIdx.x;
+    if (k2 >= plane) return;
+    const int i1 = (int)(k2 / (unsigned)g.G0), i0 = (int)(k2 - (unsigned)i1 * g.G0);
+    const long n2 = plane;
+    const double c = aux[WAVESPEEDGF * nt + NG * n2 + k2], c2 = c * c, w2 = w2d[k2];
+    const double f0 = r.f0[i0], f0p = r.f0_D0[i0], f0pp = r.f0_DD00[i0];
+    const double f1 = r.f1[i1], f1p = r.f1_D1[i1];
+    const double f2 = r.f2[k2], f2_0 = r.f2_D0[k2];
+    const double f3 = r.f3[i0], f3p = r.f3_D0[i0];
+    const double a0 = 1.0 / (f2 * f2), a2 = (f3 * f3) / (f0p * f0p), a3 = a0 / f2;
+    const double B = f3 * a3 * (f3 * (f0p * f2_0 + f0pp * f2) - f0p * f2 * f3p) / (f0p * f0p * f0p) -
+                     a2 * a3 * f2_0 - a0 * (f3 * f3) / (f0p * f0);
+    const double K[5] = {a0 * a2 * (g.invdx0 * g.invdx0), a0 * (g.invdx1 * g.invdx1),
+                         (1.0 / (f1 * f1)) / (f0 * f0) * (g.invdx2 * g.invdx2), a0 * f1p / f1 * g.invdx1,
+                         -B * g.invdx0};
 #pragma unroll
-  for (int k = 0; k < 5; k++) {
-    coef[k * n2 + k2] = K[k];
-    const double v = c2 * K[k];
-    kc64[6 * k2 + k] = v;
-    kc32[6 * k2 + k] = (float)v;
+    for (int k = 0; k < 5; k++) {
+      coef[k * n2 + k2] = K[k];
+      const double v = c2 * K[k];
+      kc64[6l * k2 + k] = v;
+      kc32[6l * k2 + k] = (float)v;
+    }
+    const double w = c2 > 0.0 ? w2 / (c2 * c2) : 0.0;
+    kc64[6l * k2 + 5] = w;
+    kc32[6l * k2 + 5] = (float)w;
+    return;
   }
-  const double w = c2 > 0.0 ? w2d[k2] / (c2 * c2) : 0.0;
-  kc64[6 * k2 + 5] = w;
-  kc32[6 * k2 + 5] = (float)w;
-}
-
-// (psi, c^2 AA^2 / 8) interleaved per point (one 16-byte load in the fused kernels); raises *bad
-// where the wave speed at an interior point differs from its value on the plane i2 = NG.
-__global__ void fold_source_kernel(GridDims g, const double *aux, double *src, int *bad) {
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x, nt = g.ntot;
-  if (p >= nt) return;
-  const int plane = g.G0 * g.G1;
-  const int i2 = (int)(p / plane), rem = (int)(p - (long)i2 * plane), i1 = rem / g.G0, i0 = rem - i1 * g.G0;
-  const double c = aux[WAVESPEEDGF * nt + p];
-  src[2 * p] = aux[PSI_BACKGROUNDGF * nt + p];
-  src[2 * p + 1] = 0.125 * (c * c) * aux[ADD_TIMES_AUUGF * nt + p];
-  const bool inside = i0 >= NG && i0 < g.N0 + NG && i1 >= NG && i1 < g.N1 + NG && i2 >= NG && i2 < g.N2 + NG;
-  if (inside && c != aux[WAVESPEEDGF * nt + (p - (long)(i2 - NG) * plane)]) *bad = 1;
+  const long k = (long)(blockIdx.x - ncoef) * 256 + threadIdx.x;
+  if (k >= (long)plane * g.N2) return;
+  const int i2 = (int)(k / plane);
+  const unsigned rem = (unsigned)(k - (long)i2 * plane), i1 = rem / (unsigned)g.G0, i0 = rem - i1 * g.G0;
+  const long p = k + (long)NG * plane;
+  const double c = aux[WAVESPEEDGF * nt + p], cq = aux[WAVESPEEDGF * nt + (long)NG * plane + rem];
+  const double psi = aux[PSI_BACKGROUNDGF * nt + p], AA = aux[ADD_TIMES_AUUGF * nt + p];
+  *(double2 *)(src + 2 * p) = make_double2(psi, 0.125 * (c * c) * AA);
+  const bool inside = i0 >= NG && i0 < (unsigned)(g.N0 + NG) && i1 >= NG && i1 < (unsigned)(g.N1 + NG);
+  if (inside && c != cq) *bad = 1;
 }
 
 void launch_tables(const GridDims &g, const rfm_struct *rfm, const double *aux, const double *w2d, double *coef64,
-                   double *kc64, float *kc32, double *src, int *bad, int *also_clear, hipStream_t st) {
-  RfmPtrs r{rfm->f0_of_xx0, rfm->f0_of_xx0__D0, rfm->f0_of_xx0__DD00, rfm->f1_of_xx1, rfm->f1_of_xx1__D1,
-            rfm->f2_of_xx0_xx1, rfm->f2_of_xx0_xx1__D0, rfm->f3_of_xx0, rfm->f3_of_xx0__D0};
-  hipLaunchKernelGGL(coef_fold_kernel, dim3((g.G0 + 63) / 64, g.G1), dim3(64), 0, st, g, r, aux, w2d, coef64, kc64,
-                     kc32, bad, also_clear);
-  hipLaunchKernelGGL(fold_source_kernel, dim3((unsigned)((g.ntot + 255) / 256)), dim3(256), 0, st, g, aux, src, bad);
+                   double *kc64, float *kc32, double *src, int *bad, hipStream_t st) {
+  const long plane = (long)g.G0 * g.G1;
+  const unsigned ncoef = (unsigned)((plane + 255) / 256), nsrc = (unsigned)((plane * g.N2 + 255) / 256);
+  hipLaunchKernelGGL(tables_kernel, dim3(ncoef + nsrc), dim3(256), 0, st, g, exact_rfm(rfm), aux, w2d, coef64, kc64,
+                     kc32, src, bad, ncoef);
 }
 
 // ---------------------------------------------------------------------------------------

@@ -31,6 +31,10 @@
 //   launch 2 (stages 3+4): in = k_odd, y = A_j, rt; writes A_(1-j) = y + (rt + dt/3 k3) + dt/6 k4
 // (Storing stage 4's u from launch 1, so that launch 2 reads two arrays instead of three on its
 // boxes and i2 arms, measured no faster: launch 2 gained what launch 1 lost.)
+// (HOME, the drop-in step: launch 1 also copies y to k_even_gfs, launch 2 reads it there and writes
+// y_n_gfs in place, with every parity image, where the resident solver only needs those in the
+// interior phi planes: 24.0 us for the two launches at 128x128x16, against 21.0 and a pass of 5.2 that
+// copied the state back and filled its ghost planes.)
 // y_n is never overwritten within its step, so when stage 1's fused residual check (reduced by
 // the second launch's block 0) ends the solve, A_j still holds the state it checked.
 #include <hip/hip_runtime.h>
@@ -148,7 +152,7 @@ constexpr int bc2_lds() {
   return 2 * NRB * NT + NR1 * (24 + 10 + 24 + 2 + 12) + TYB * (10 + 30 + 8 + 10 + 2 + 12) + NRPYELL_FD_TABLE;
 }
 
-template <typename T, int PAIR, int TX, int PL, int MODE>
+template <typename T, int PAIR, int TX, int PL, int MODE, bool HOME>
 __device__ __forceinline__ void interior2_body(const SubstepArgs<T> &a, const int tile, const int pgroup,
                                                const unsigned bid, const unsigned nblk, T *lds, double *s_red) {
   constexpr int S0 = PAIR;
@@ -324,10 +328,20 @@ __device__ __forceinline__ void interior2_body(const SubstepArgs<T> &a, const in
       }
       st32(a.out, p, ou);
       st32(a.out, nt + p, ov);
-      for_each_image_in_planes(g, i0, i1, i2, [&](long d) {
+      if (HOME && PAIR == 1) {
+        st32(a.copy, p, uu);
+        st32(a.copy, nt + p, vv);
+      }
+      auto image = [&](long d) {
         st32(a.out, (unsigned)d, ou);
         st32(a.out, nt + (unsigned)d, ov);
-      });
+        if (HOME && PAIR == 1) {
+          st32(a.copy, (unsigned)d, uu);
+          st32(a.copy, nt + (unsigned)d, vv);
+        }
+      };
+      if (HOME && PAIR == 3) for_each_image(g, i0, i1, i2, image);
+      else for_each_image_in_planes(g, i0, i1, i2, image);
     }
   }
 
@@ -379,7 +393,7 @@ __device__ __forceinline__ void r1_stencil_point(int t, int ilast, int &e, int &
   }
 }
 
-template <typename T, int PAIR, int MODE>
+template <typename T, int PAIR, int MODE, bool HOME>
 __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, const int plane, T *lds) {
   constexpr int S0 = PAIR;
   constexpr int NT = NRPYELL_BLOCK, TYB = NRPYELL_PAIR_BC_ROWS;
@@ -614,7 +628,13 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
         o = y + fma((T)(1.0 / 6.0), dt * rhs, rt);
       }
       st32(a.out, gf * nt + p, o);
-      for_each_image_in_planes(g, ilast + pt, row, i2, [&](long d) { st32(a.out, gf * nt + (unsigned)d, o); });
+      if (HOME && PAIR == 1) st32(a.copy, gf * nt + p, y);
+      auto image = [&](long d) {
+        st32(a.out, gf * nt + (unsigned)d, o);
+        if (HOME && PAIR == 1) st32(a.copy, gf * nt + (unsigned)d, y);
+      };
+      if (HOME && PAIR == 3) for_each_image(g, ilast + pt, row, i2, image);
+      else for_each_image_in_planes(g, ilast + pt, row, i2, image);
     }
   }
 }
@@ -622,7 +642,7 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
 // One configuration. Without a placement table: the nbc_rows*N2 BC blocks first, then the
 // interior blocks in XCD-aware order. With one (ord.n == gridDim.x): workgroup L is logical block
 // ord.q[L], the BC blocks being logical 0 .. nb-1.
-template <typename T, int PAIR, int TX, int PL, int MODE>
+template <typename T, int PAIR, int TX, int PL, int MODE, bool HOME = false>
 __global__ void __launch_bounds__(NRPYELL_BLOCK, 3) substep2_kernel(SubstepArgs<T> a, const BlockOrder ord) {
   constexpr int NL = interior2_lds<TX, PL>() > bc2_lds() ? interior2_lds<TX, PL>() : bc2_lds();
   __shared__ T lds[NL];
@@ -633,12 +653,12 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, 3) substep2_kernel(SubstepArgs<
   const unsigned L = ordered ? v : blockIdx.x;
   if (L < nb) {
     const unsigned pln = div_by(L, a.nbc_mul);
-    bc2_body<T, PAIR, MODE>(a, (int)(L - pln * (unsigned)a.nbc_rows), (int)pln, lds);
+    bc2_body<T, PAIR, MODE, HOME>(a, (int)(L - pln * (unsigned)a.nbc_rows), (int)pln, lds);
     return;
   }
   const unsigned q = ordered ? L - nb : xcd_logical(L - nb, ni), ng = (unsigned)(a.g.N2 / PL);
   const unsigned tile = div_by(q, a.ng_mul);
-  interior2_body<T, PAIR, TX, PL, MODE>(a, (int)tile, (int)(q - tile * ng), q, ni, lds, s_red);
+  interior2_body<T, PAIR, TX, PL, MODE, HOME>(a, (int)tile, (int)(q - tile * ng), q, ni, lds, s_red);
 }
 
 // Many configurations (uneven grids) in one launch, as substep_batched_kernel does for one
@@ -660,12 +680,12 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, 3)
   const unsigned local = q - block_first[c], nb = (unsigned)(a.nbc_rows * a.g.N2);
   if (local < nb) {
     const unsigned pln = div_by(local, a.nbc_mul);
-    bc2_body<double, PAIR, MODE>(a, (int)(local - pln * (unsigned)a.nbc_rows), (int)pln, lds);
+    bc2_body<double, PAIR, MODE, false>(a, (int)(local - pln * (unsigned)a.nbc_rows), (int)pln, lds);
     return;
   }
   const unsigned li = local - nb, ng = (unsigned)(a.g.N2 / PL);
   const unsigned tile = div_by(li, a.ng_mul);
-  interior2_body<double, PAIR, TX, PL, MODE>(a, (int)tile, (int)(li - tile * ng), li, a.ntile0 * a.ntile1 * ng, lds, s_red);
+  interior2_body<double, PAIR, TX, PL, MODE, false>(a, (int)tile, (int)(li - tile * ng), li, a.ntile0 * a.ntile1 * ng, lds, s_red);
 }
 
 template <int V>
@@ -736,3 +756,30 @@ void launch_substep_pair(const SubstepArgs<T> &a, int first_stage, hipStream_t s
 }
 template void launch_substep_pair<double>(const SubstepArgs<double> &, int, hipStream_t, const BlockOrder *);
 template void launch_substep_pair<float>(const SubstepArgs<float> &, int, hipStream_t, const BlockOrder *);
+
+template <int PL, int MODE>
+static void step_in_place(SubstepArgs<double> &a, double *y_n, double *k_odd, double *copy, hipStream_t st,
+                          const BlockOrder &o) {
+  dim3 grd(a.nbc_rows * a.g.N2 + a.ntile0 * a.ntile1 * (a.g.N2 / PL)), blk(NRPYELL_BLOCK);
+  a.in = a.yn = y_n;
+  a.out = k_odd;
+  a.copy = copy;
+  hipLaunchKernelGGL((substep2_kernel<double, 1, 32, PL, MODE, true>), grd, blk, 0, st, a, o);
+  a.in = k_odd;
+  a.yn = copy;
+  a.out = y_n;
+  hipLaunchKernelGGL((substep2_kernel<double, 3, 32, PL, MODE, true>), grd, blk, 0, st, a, o);
+}
+
+void launch_step_in_place(SubstepArgs<double> a, double *y_n, double *k_odd, double *copy, hipStream_t st,
+                          const BlockOrder *ord) {
+  static const BlockOrder none{};
+  const BlockOrder &o = ord ? *ord : none;
+  if (a.g.N2 >= 6) {
+    if (a.pl == 2) step_in_place<2, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
+    else step_in_place<1, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
+  } else {
+    if (a.pl == 2) step_in_place<2, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
+    else step_in_place<1, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
+  }
+}
