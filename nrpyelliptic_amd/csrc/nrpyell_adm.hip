@@ -3,14 +3,14 @@
 // (NRPyEllipticET_conformally_flat_BBH_Initialize_ADMBase.c:5-200), and the optimum damping
 // parameter of the ET relaxation driver (conformally_flat_BBH_set_optimum_eta_damping.c:3-27).
 //
-// One thread per Cartesian point: orbital-plane permutation and shift, the closed-form inverse
-// of the SinhSymTP map, a tensor-product Lagrange interpolation of u from the grid (the
-// molecule placement of the Cactus AEILocalInterp operator the thorn calls), the Bowen-York
-// ADM fields. u (4 MB at 128x128x16) stays in L2/MALL across the molecule reads; the 17
-// outputs are written once, coalesced.
+// Per Cartesian point: orbital-plane permutation and shift, the closed-form inverse of the
+// SinhSymTP map, a tensor-product Lagrange interpolation of u from the grid (the molecule placement of
+// the Cactus AEILocalInterp operator the thorn calls), the Bowen-York ADM fields. u (4 MB at
+// 128x128x16) stays in L2/MALL across the molecule reads; the 17 outputs are written once, coalesced.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <mutex>
 #include <string>
 
 #include "nrpyell_common.h"
@@ -28,7 +28,8 @@ struct AdmArgs {
   const double *u, *x, *y, *z;
   double *out[NRPYELL_ADM_NOUT];
   long n;
-  int *err;  // 1: NaN coordinate after the epsilon retry, 2: point outside the grid
+  int *err;  // [0] set: NaN coordinate after the epsilon retry; [1] set: point outside the grid
+  double sinh_1w;  // sinh(1 / SINHWAA)
 };
 
 // conformally_flat_BBH_get_xx_from_xyz.c:6-20 (the closed-form inverse of the SinhSymTP map).
@@ -38,7 +39,7 @@ __device__ inline void xx_from_xyz(const AdmArgs &a, const double X[3], double x
   const double Q = sqrt(-4 * (X[2] * X[2]) * b2 + b * b * b * b + 2 * b2 * R2 + R2 * R2);
   const double ib2 = 1.0 / b2;
   const double sgn = (double)((X[2] > 0) - (X[2] < 0));
-  xx[0] = a.SINHWAA * asinh(M_SQRT1_2 * sqrt(-b2 + R2 + Q) * sinh(1.0 / a.SINHWAA) / a.AMAX);
+  xx[0] = a.SINHWAA * asinh(M_SQRT1_2 * sqrt(-b2 + R2 + Q) * a.sinh_1w / a.AMAX);
   xx[1] = acos(0.99999999 * M_SQRT1_2 * sqrt(R2 * ib2 - Q * ib2 + 1) * sgn);
   xx[2] = atan2(X[1], X[0]);
 }
@@ -71,11 +72,42 @@ __device__ inline bool axis_weights(int n, double origin, double delta, double x
   return true;
 }
 
+// two neighbouring doubles, 8-byte aligned: one 16-byte load
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// psi^n, the lapse. For the default n = -2 the square's rounding error and one Newton step on the
+// quotient give the correctly rounded value to within 0.01 ulp or so in 10 instructions; the general
+// power takes some 200.
+__device__ inline double psi_power(double x, double n) {
+  if (n == -2.0 && x > 1e-100 && x < 1e100) {
+    const double s = x * x, e = fma(x, x, -s), r = 1.0 / s;
+    return fma(r, fma(-s, r, 1.0) - e * r, r);
+  }
+  return pow(x, n);
+}
+
+// A block is one wave and 64 points. The closed forms run one point per thread; the molecule sums run
+// four lanes per point, 16 points per pass, because the gather of u is bound by the number of cache
+// lines the vector loads touch (the texture data unit is busy 86 % of the time): a lane reads two
+// neighbouring values (16 bytes) of a row, so one load fetches the row of 16 points from 24 lines
+// where a point per lane needs three loads of 47 lines each. The lanes take the weights from LDS and
+// sum over xx1 and xx2 for their two columns; the columns are added last. The 17 outputs, 285 MB at 2.1
+// million points, go out with streaming stores so that they do not evict u from L2. 2.1 million points,
+// order 4: 150 us (point per lane, ordinary stores: 196 us; four lanes but ordinary stores 183 us;
+// 256-thread blocks 157 us); the closed forms and the stores alone take 98 us.
+constexpr int ADM_T = 64;
+
 template <int ORDER>
-__global__ void __launch_bounds__(256) admbase_kernel(AdmArgs a) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= a.n) return;
-  const double px = a.x[i], py = a.y[i], pz = a.z[i];
+__global__ void __launch_bounds__(ADM_T) admbase_kernel(AdmArgs a) {
+  constexpr int NP = ORDER + 1;
+  __shared__ double s_w[3][NP][ADM_T];
+  __shared__ unsigned s_base[ADM_T];
+  double *s_u = s_w[0][0];  // a point's sum replaces its first weight, which only its own lanes read
+  const int tid = threadIdx.x;
+  const long i = (long)blockIdx.x * ADM_T + tid;
+  const bool on = i < a.n;
+  const long ic = on ? i : a.n - 1;
+  const double px = a.x[ic], py = a.y[ic], pz = a.z[ic];
   const double s[3] = {px - a.shift[0], py - a.shift[1], pz - a.shift[2]};
   // (x,y,z)_NRPy = (y,z,x)_ETK for the "xy" orbital plane
   double X[3] = {a.xy ? s[1] : s[0], a.xy ? s[2] : s[1], a.xy ? s[0] : s[2]};
@@ -87,51 +119,64 @@ __global__ void __launch_bounds__(256) admbase_kernel(AdmArgs a) {
     X[2] += a.eps;
     xx_from_xyz(a, X, xx);
   }
-  double w[3][ORDER + 1];
-  int f[3];
   bool ok = !isnan(xx[0] * xx[1] * xx[2]);
   if (!ok) {
-    atomicMax(a.err, 1);
+    a.err[0] = 1;
   } else {
+    int f[3];
 #pragma unroll
-    for (int d = 0; d < 3; d++) ok = ok && axis_weights<ORDER>(a.dims[d], a.origin[d], a.delta[d], xx[d], f[d], w[d]);
-    if (!ok) atomicMax(a.err, 2);
+    for (int d = 0; d < 3; d++) {
+      double w[NP];
+      ok = ok && axis_weights<ORDER>(a.dims[d], a.origin[d], a.delta[d], xx[d], f[d], w);
+#pragma unroll
+      for (int m = 0; m < NP; m++) s_w[d][m][tid] = w[m];
+    }
+    if (!ok) a.err[1] = 1;
+    s_base[tid] =
+        ok ? (unsigned)f[0] + (unsigned)a.dims[0] * ((unsigned)f[1] + (unsigned)a.dims[1] * (unsigned)f[2]) : 0;
   }
+  if (!ok) s_base[tid] = 0;  // such a point's sum is not used
+  __syncthreads();
+  {
+    const int lane = tid & 63, col = 2 * (lane & 3);  // this lane's columns col, col + 1 of the molecule
+    const long d0 = a.dims[0], d01 = d0 * a.dims[1];
+#pragma unroll 1
+    for (int pass = 0; pass < 4; pass++) {
+      const int pt = (tid & ~63) + 16 * pass + (lane >> 2);
+      double v = 0.0;
+      if (col < NP) {
+        const double *p = a.u + s_base[pt] + col;
+        double w1[NP], acc0 = 0.0, acc1 = 0.0;
+#pragma unroll
+        for (int j = 0; j < NP; j++) w1[j] = s_w[1][j][pt];
+#pragma unroll 1
+        for (int k = 0; k < NP; k++) {
+          double2u r[NP];
+#pragma unroll
+          for (int j = 0; j < NP; j++) r[j] = *(const double2u *)(p + k * d01 + j * d0);
+          double t0 = 0.0, t1 = 0.0;
+#pragma unroll
+          for (int j = 0; j < NP; j++) {
+            t0 = fma(w1[j], r[j].x, t0);
+            t1 = fma(w1[j], r[j].y, t1);
+          }
+          const double w2 = s_w[2][k][pt];
+          acc0 = fma(w2, t0, acc0);
+          acc1 = fma(w2, t1, acc1);
+        }
+        v = s_w[0][col][pt] * acc0;
+        if (col + 1 < NP) v = fma(s_w[0][col + 1][pt], acc1, v);
+      }
+      v += __shfl_xor(v, 1, 64);
+      v += __shfl_xor(v, 2, 64);
+      if (col == 0) s_u[pt] = v;
+    }
+  }
+  __syncthreads();
+  if (!on) return;
   double v[NRPYELL_ADM_NOUT];
   if (ok) {
-    // sum in the order k (xx2), j (xx1), i (xx0 contiguous rows)
-    double acc = 0.0;
-    if constexpr (ORDER >= 5) {
-      // one xx2 plane of loads in flight at a time: with the loads of all (ORDER+1)^3 values
-      // hoisted the kernel needs 256 VGPRs and spills (order 6: 252 of them)
-#pragma unroll 1
-      for (int k = 0; k <= ORDER; k++) {
-        double a1 = 0.0;
-        for (int j = 0; j <= ORDER; j++) {
-          const double *row =
-              a.u + (long)f[0] + (long)a.dims[0] * ((long)(f[1] + j) + (long)a.dims[1] * (long)(f[2] + k));
-          double a0 = 0.0;
-#pragma unroll
-          for (int ii = 0; ii <= ORDER; ii++) a0 += w[0][ii] * row[ii];
-          a1 += w[1][j] * a0;
-        }
-        acc += w[2][k] * a1;
-      }
-    } else {
-      for (int k = 0; k <= ORDER; k++) {
-        double a1 = 0.0;
-        for (int j = 0; j <= ORDER; j++) {
-          const double *row =
-              a.u + (long)f[0] + (long)a.dims[0] * ((long)(f[1] + j) + (long)a.dims[1] * (long)(f[2] + k));
-          double a0 = 0.0;
-#pragma unroll
-          for (int ii = 0; ii <= ORDER; ii++) a0 += w[0][ii] * row[ii];
-          a1 += w[1][j] * a0;
-        }
-        acc += w[2][k] * a1;
-      }
-    }
-    const double uu = acc;
+    const double uu = s_u[tid];
     // conformally_flat_BBH_compute_ADM_Cartesian_quantities_from_uu.c:36-103 and the lapse
     // choices (..._lapse_power_of_psi_initial_data.c:16-35, ..._lapse_averaged_initial_data.c:18-41),
     // at the ETK point itself
@@ -142,7 +187,7 @@ __global__ void __launch_bounds__(256) admbase_kernel(AdmArgs a) {
     const double psi = ((uu + 1.0) + h[0]) + h[1];
     const double psi4 = psi * psi * psi * psi, ipsi2 = 1.0 / (psi * psi);
     v[0] = uu;
-    v[1] = a.lapse ? 0.5 * (1.0 - F) / (F + 1.0) + 0.5 : pow((F + uu) + 1.0, a.lapse_n);
+    v[1] = a.lapse ? 0.5 * (1.0 - F) / (F + 1.0) + 0.5 : psi_power((F + uu) + 1.0, a.lapse_n);
     v[2] = v[3] = v[4] = 0.0;
     v[5] = psi4; v[6] = 0.0; v[7] = 0.0; v[8] = psi4; v[9] = 0.0; v[10] = psi4;
     v[11] = ipsi2 * A[0][0]; v[12] = ipsi2 * A[0][1]; v[13] = ipsi2 * A[0][2];
@@ -152,8 +197,21 @@ __global__ void __launch_bounds__(256) admbase_kernel(AdmArgs a) {
     for (int c = 0; c < NRPYELL_ADM_NOUT; c++) v[c] = __builtin_nan("");
   }
 #pragma unroll
-  for (int c = 0; c < NRPYELL_ADM_NOUT; c++) a.out[c][i] = v[c];
+  for (int c = 0; c < NRPYELL_ADM_NOUT; c++) __builtin_nontemporal_store(v[c], a.out[c] + i);
 }
+
+// The two error flags of a call: pinned host memory that the kernel writes and the host reads after
+// it, without an allocation, a clearing or a copy per call. One pair for the process (portable: any
+// device writes it), held with the lock from clearing to reading.
+std::mutex g_err_mu;
+struct ErrFlags {
+  int *host = nullptr, *dev = nullptr;
+  ErrFlags() {
+    HIPCHK(hipHostMalloc((void **)&host, 2 * sizeof(int),
+                         hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
+    HIPCHK(hipHostGetDevicePointer((void **)&dev, host, 0));
+  }
+};
 
 }  // namespace
 
@@ -240,11 +298,13 @@ extern "C" int nrpyell_Initialize_ADMBase(const griddata_struct *gd, const nrpye
     a.z = z;
     for (int c = 0; c < NRPYELL_ADM_NOUT; c++) a.out[c] = outs[c];
     a.n = n;
-    DevBuf<int> errb(1);
-    int *err = errb.p;
-    HIPCHK(hipMemset(err, 0, sizeof(int)));
-    a.err = err;
-    const dim3 grd((unsigned)((n + 255) / 256)), blk(256);
+    a.sinh_1w = sinh(1.0 / p->SINHWAA);
+    std::lock_guard<std::mutex> lk(g_err_mu);
+    static ErrFlags flags;
+    volatile int *err = flags.host;
+    err[0] = err[1] = 0;
+    a.err = flags.dev;
+    const dim3 grd((unsigned)((n + ADM_T - 1) / ADM_T)), blk(ADM_T);
     switch (opt->interpolation_order) {
       case 1: hipLaunchKernelGGL(admbase_kernel<1>, grd, blk, 0, 0, a); break;
       case 2: hipLaunchKernelGGL(admbase_kernel<2>, grd, blk, 0, 0, a); break;
@@ -254,14 +314,13 @@ extern "C" int nrpyell_Initialize_ADMBase(const griddata_struct *gd, const nrpye
       default: hipLaunchKernelGGL(admbase_kernel<4>, grd, blk, 0, 0, a); break;
     }
     HIPCHK(hipGetLastError());
-    int herr = 0;
-    HIPCHK(hipMemcpy(&herr, err, sizeof(int), hipMemcpyDeviceToHost));
-    if (herr == 1) {
+    HIPCHK(hipStreamSynchronize(0));
+    if (err[1] == 0 && err[0] != 0) {
       set_last_error("NAN found in (xx0,xx1,xx2) after moving the point by NRPy_epsilon; consider increasing "
                      "NRPy_epsilon");
       return NRPYELL_ENAN;
     }
-    if (herr == 2) {
+    if (err[1] != 0) {
       set_last_error("Interpolation point outside the NRPyElliptic grid");
       return NRPYELL_EINVAL;
     }
