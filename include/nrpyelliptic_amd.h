@@ -267,9 +267,9 @@ typedef struct {
   double integration_radius;  /* L2 mask radius, 100 in the reference driver (main.c:150) */
   int tile_i0;            /* i0 width of the fused substep kernel's 256-thread tile: 16, 32
                              or 64 (0 = default); the i1 height is 256 / tile_i0            */
-  int planes;             /* i2 planes per thread: 1, or 2 with tile_i0 32/64 (0 = 1 where the
-                             tile allows no 2, or the grid is so small that one-plane blocks
-                             get a CU each; else 2)                                         */
+  int planes;             /* i2 planes per thread: 1, or 2 with tile_i0 32/64; 0 = chosen by the
+                             grid's size (1 where those blocks get a CU each or the tile
+                             allows no 2; 4 on large grids and batches; else 2)             */
   int outer_bc;           /* NRPYELL_OUTER_BC_RADIATION: apply_bcs_outerradiation_and_inner;
                              NRPYELL_OUTER_BC_SOMMERFELD6: the Einstein Toolkit thorn's BC
                              (nrpyell_apply_bcs_sommerfeld with f_infinity 0, falloff 3)      */

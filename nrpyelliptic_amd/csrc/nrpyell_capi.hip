@@ -1060,8 +1060,28 @@ extern "C" void nrpyell_default_options(nrpyell_solve_options *o) {
   o->substeps_per_launch = 0;
 }
 
-extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell_solve_options *opt,
-                                     nrpyell_solver **out) {
+// Four planes per thread (two-substep kernel, 32-wide tiles): the window of planes per thread is 14
+// for 4 points instead of 12 for 2, a quarter fewer vector loads, whose rate bounds the kernel once
+// many blocks hide its latencies (texture data unit 66 / 76 % busy at 256x256x32); but it takes 168 / 241
+// registers, so two of its blocks fit a CU where three of the others do. It pays where the blocks
+// make one full round of two per CU or many rounds. us per RK4 step, two / four planes, by four-plane
+// blocks: 256 (128x128x16) 20.8 / 22.3, 320 (160x128x16) 22.5 / 24.5, 476 (200x130x16) 33.0 / 32.0, 512
+// (256x128x16) 34.6 / 31.5, 640 (256x160x16) 40.6 / 41.4, 800 (160x160x32) 51.4 / 51.5, 1024 (256x256x16)
+// 56.5 / 52.4, 2048 (256x256x32) 101.2 / 96.1, 4096 (512x256x32) 240 / 212. In a batch the BC blocks and
+// the members' ragged tiles fill the gaps: 2 members (328 blocks) 32.4 / 31.2, 8 (1488) 87.2 / 81.0,
+// 16 (2980) 178 / 155, 48 661 / 574.
+static bool four_planes_allowed(const GridDims &g, int tx, const nrpyell_solve_options &o) {
+  return tx == 32 && g.N2 % 4 == 0 && o.substeps_per_launch != 1;
+}
+static bool four_planes_pay(long blocks, int ncu) {
+  return 4 * blocks >= 15l * ncu || (4 * blocks >= 7l * ncu && blocks <= 2l * ncu);
+}
+static bool four_planes_pay_in_batch(long blocks, int ncu) { return 4 * blocks >= 5l * ncu; }
+
+// auto_planes: planes per thread where the caller's options leave them open; 0: chosen for this grid
+// alone on the GPU
+static int make_solver(griddata_struct *gd, REAL dt, const nrpyell_solve_options *opt, int auto_planes,
+                       nrpyell_solver **out) {
   return api_call([&]() -> int {
     std::lock_guard<std::mutex> lk(g_mu);
     auto s = std::make_unique<nrpyell_solver>();
@@ -1108,17 +1128,21 @@ extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell
     s->ntile0 = (g.N0 + tx - 1) / tx;
     s->ntile1 = (g.N1 + ty - 1) / ty;
     int pl = s->opt.planes;
-    if (pl <= 0) {
+    if (pl != 1 && !(pl == 2 && tx >= 32) && pl > 0) {
+      set_last_error("planes must be 1, or 2 with tile_i0 32 or 64");
+      return NRPYELL_EINVAL;
+    }
+    if (pl <= 0 && auto_planes > 0) {
+      pl = auto_planes;
+    } else if (pl <= 0) {
       // Two planes per thread share the coefficients and most of the phi window; one plane leaves half
       // the work per block, which is faster while those blocks still get a CU each (us per RK4 step,
       // one / two planes: 16x16x6 13.7 / 14.6, 64x64x4 13.3 / 13.6, 64x64x8 14.1 / 14.2; past that
       // 64x64x16 16.8 / 15.1, 96x96x8 16.9 / 15.2, 128x128x16 23.5 / 20.2).
       const long blocks = (long)g.N2 * (s->ntile0 * s->ntile1 + (g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS);
       pl = tx >= 32 && blocks > cu_count() ? 2 : 1;
-    }
-    if (pl != 1 && !(pl == 2 && tx >= 32)) {
-      set_last_error("planes must be 1, or 2 with tile_i0 32 or 64");
-      return NRPYELL_EINVAL;
+      if (four_planes_allowed(g, tx, s->opt) && four_planes_pay((long)s->ntile0 * s->ntile1 * (g.N2 / 4), cu_count()))
+        pl = 4;
     }
     s->tx = tx;
     s->pl = pl;
@@ -1173,7 +1197,7 @@ extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell
       return NRPYELL_EINVAL;
     }
     const long nblk_res = (long)((g.N0 + 63) / 64) * ((g.N1 + 3) / 4) * g.N2;
-    const long nblk_sub = (long)s->ntile0 * s->ntile1 * (g.N2 / pl);
+    const long nblk_sub = (long)s->ntile0 * s->ntile1 * (g.N2 / (pl < 2 ? pl : 2));
     s->partial = dalloc<double>(nblk_res > nblk_sub ? nblk_res : nblk_sub);
     s->l2_out = dalloc<double>(1);
     s->dstate = dalloc<SolverDeviceState>(1);
@@ -1184,6 +1208,11 @@ extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell
     *out = s.release();
     return NRPYELL_OK;
   });
+}
+
+extern "C" int nrpyell_solver_create(griddata_struct *gd, REAL dt, const nrpyell_solve_options *opt,
+                                     nrpyell_solver **out) {
+  return make_solver(gd, dt, opt, 0, out);
 }
 
 extern "C" int nrpyell_solver_destroy(nrpyell_solver *s) {
@@ -1491,13 +1520,17 @@ extern "C" int nrpyell_solver_time_substep(nrpyell_solver *s, int stage, int n, 
       (void)hipEventDestroy(e1);
       return NRPYELL_OK;
     }
-    // stage 0 = stage 1 with the fused residual-L2 check (the form the solver runs)
+    // stage 0 = stage 1 with the fused residual-L2 check (the form the one-substep path runs)
     const bool fuse = stage == 0;
     if (fuse) stage = 1;
     // the kernels write y_n only in stage 4; time on scratch copies so the state is untouched
     SubstepArgs<double> a =
         s->args<double>(stage, f.y_n_gfs, f.k_odd_gfs, f.k_even_gfs, f.y_nplus1_running_total_gfs, s->src64,
                         s->kc64, s->geo64);
+    if (a.pl == 4) {  // the one-substep kernel has one and two planes
+      a.pl = 2;
+      a.ng_mul = div_mul((unsigned)(s->g.N2 / 2));
+    }
     if (fuse) {
       a.l2_partial = s->partial;
       a.state = s->dstate;
@@ -1790,14 +1823,29 @@ extern "C" int nrpyell_batch_create(griddata_struct **gds, const double *dts, co
       set_last_error("the batched solver stops every configuration by NRPYELL_STOP_EVERY_STEP");
       return NRPYELL_EINVAL;
     }
-    for (int k = 0; k < n; k++) {
+    // planes per thread of the members that leave them open: the launches are the whole batch's, so
+    // no one-plane blocks for a small grid's sake, and four planes by the blocks of all members
+    auto options_of = [&](int k) {
       nrpyell_solve_options o = b->opt;
       o.tile_i0 = tile_i0 ? tile_i0[k] : b->opt.tile_i0;
       o.planes = planes ? planes[k] : b->opt.planes;
-      // the other configurations fill the GPU: no one-plane blocks for a small one's sake
-      if (o.planes <= 0) o.planes = o.tile_i0 == 16 ? 1 : 2;
+      return o;
+    };
+    auto four = [&](int k) {
+      const nrpyell_solve_options o = options_of(k);
+      return o.planes <= 0 && four_planes_allowed(dims_from_params(&gds[k]->params), o.tile_i0 > 0 ? o.tile_i0 : 32, o);
+    };
+    long blocks4 = 0;
+    for (int k = 0; k < n; k++) {
+      const GridDims g = dims_from_params(&gds[k]->params);
+      const int ty = NRPYELL_BLOCK / 32;
+      if (four(k)) blocks4 += (long)((g.N0 + 31) / 32) * ((g.N1 + ty - 1) / ty) * (g.N2 / 4);
+    }
+    const bool pay = four_planes_pay_in_batch(blocks4, cu_count());
+    for (int k = 0; k < n; k++) {
+      const nrpyell_solve_options o = options_of(k);
       nrpyell_solver *s = nullptr;
-      const int rc = nrpyell_solver_create(gds[k], dts[k], &o, &s);
+      const int rc = make_solver(gds[k], dts[k], &o, four(k) && pay ? 4 : o.tile_i0 == 16 ? 1 : 2, &s);
       if (rc != NRPYELL_OK) return rc;
       b->solvers.push_back(s);
     }

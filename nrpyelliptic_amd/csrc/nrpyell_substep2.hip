@@ -642,8 +642,11 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
 // One configuration. Without a placement table: the nbc_rows*N2 BC blocks first, then the
 // interior blocks in XCD-aware order. With one (ord.n == gridDim.x): workgroup L is logical block
 // ord.q[L], the BC blocks being logical 0 .. nb-1.
+// Blocks per CU: three, or two where a thread's four planes need more than 168 registers.
+constexpr int pair_occupancy(int pl) { return pl == 4 ? 2 : 3; }
+
 template <typename T, int PAIR, int TX, int PL, int MODE, bool HOME = false>
-__global__ void __launch_bounds__(NRPYELL_BLOCK, 3) substep2_kernel(SubstepArgs<T> a, const BlockOrder ord) {
+__global__ void __launch_bounds__(NRPYELL_BLOCK, pair_occupancy(PL)) substep2_kernel(SubstepArgs<T> a, const BlockOrder ord) {
   constexpr int NL = interior2_lds<TX, PL>() > bc2_lds() ? interior2_lds<TX, PL>() : bc2_lds();
   __shared__ T lds[NL];
   __shared__ double s_red[NRPYELL_BLOCK / 64];
@@ -667,7 +670,7 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, 3) substep2_kernel(SubstepArgs<
 // converged returns at once (its own done flag). Block 0 of a configuration's interior blocks
 // of the stages-3+4 launch reduces that configuration's residual partials.
 template <int PAIR, int TX, int PL, int MODE>
-__global__ void __launch_bounds__(NRPYELL_BLOCK, 3)
+__global__ void __launch_bounds__(NRPYELL_BLOCK, pair_occupancy(PL))
     substep2_batched_kernel(const SubstepArgs<double> *__restrict__ cfgs, const int *__restrict__ block_cfg,
                             const int *__restrict__ block_first) {
   constexpr int NL = interior2_lds<TX, PL>() > bc2_lds() ? interior2_lds<TX, PL>() : bc2_lds();
@@ -707,6 +710,10 @@ template <int PAIR, int MODE>
 static void launch_pair_batched(const SubstepArgs<double> *cfgs, const int *block_cfg, const int *block_first,
                                 int nblocks, int tx, int pl, hipStream_t st) {
   dim3 grd(nblocks), blk(NRPYELL_BLOCK);
+  if (pl == 4) {
+    hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 32, 4, MODE>), grd, blk, 0, st, cfgs, block_cfg, block_first);
+    return;
+  }
   if (pl == 2) {
     switch (tx) {
       case 64: hipLaunchKernelGGL((substep2_batched_kernel<PAIR, 64, 2, MODE>), grd, blk, 0, st, cfgs, block_cfg, block_first); break;
@@ -733,6 +740,10 @@ void launch_substep_pair_batched(const SubstepArgs<double> *cfgs, const int *blo
 template <typename T, int PAIR, int MODE>
 static void launch_pair(const SubstepArgs<T> &a, hipStream_t st, const BlockOrder &o) {
   dim3 grd(a.nbc_rows * a.g.N2 + a.ntile0 * a.ntile1 * (a.g.N2 / a.pl)), blk(NRPYELL_BLOCK);
+  if (a.pl == 4) {
+    hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 4, MODE>), grd, blk, 0, st, a, o);
+    return;
+  }
   if (a.pl == 2) {
     switch (a.tx) {
       case 64: hipLaunchKernelGGL((substep2_kernel<T, PAIR, 64, 2, MODE>), grd, blk, 0, st, a, o); break;
@@ -776,10 +787,12 @@ void launch_step_in_place(SubstepArgs<double> a, double *y_n, double *k_odd, dou
   static const BlockOrder none{};
   const BlockOrder &o = ord ? *ord : none;
   if (a.g.N2 >= 6) {
-    if (a.pl == 2) step_in_place<2, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
+    if (a.pl == 4) step_in_place<4, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
+    else if (a.pl == 2) step_in_place<2, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
     else step_in_place<1, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
   } else {
-    if (a.pl == 2) step_in_place<2, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
+    if (a.pl == 4) step_in_place<4, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
+    else if (a.pl == 2) step_in_place<2, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
     else step_in_place<1, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
   }
 }
