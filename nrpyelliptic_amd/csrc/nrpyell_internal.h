@@ -225,7 +225,7 @@ void launch_l2_weights(const GridDims &g, const L2WeightParams &q, const double 
 void launch_l2_finalize_weights(const double *partial, long npart, const double *w2d, long nw, int n2,
                                 double *log10_out, hipStream_t st);
 void launch_l2_finalize(const double *partial, long npart, double volume, SolverDeviceState *dst, int steps_per_check,
-                        double target, double *log10_out, hipStream_t st);
+                        double target, double *log10_out, hipStream_t st, int *signal = nullptr);
 void launch_inner_gather(long nt, int n, const int *dst, const int *src, const int8_t *par0, double *gfs,
                          hipStream_t st);
 void launch_radiation_rows(const GridDims &g, int n, const RadLayers &L, const double *gfs, double *rhs, double c_u,

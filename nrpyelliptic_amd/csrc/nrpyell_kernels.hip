@@ -388,10 +388,11 @@ __global__ void __launch_bounds__(256) l2_partial_kernel(GridDims g, const doubl
 }
 
 // Fixed-order sum of the partials by one block; writes log10(1e-16+sqrt(S/V)) and, when `st`
-// is given, updates the solver convergence state.
+// is given, updates the solver convergence state. `signal`: a flag in host memory, set when all of it is
+// stored.
 __global__ void __launch_bounds__(256) l2_finalize_kernel(const double *partial, long npart, double volume,
                                                           SolverDeviceState *st, int steps_per_check,
-                                                          double target, double *log10_out) {
+                                                          double target, double *log10_out, int *signal) {
   if (st && st->done) return;
   double acc = 0.0;
   for (long i = threadIdx.x; i < npart; i += 256) acc += partial[i];
@@ -406,6 +407,10 @@ __global__ void __launch_bounds__(256) l2_finalize_kernel(const double *partial,
     if (st) {
       st->steps += steps_per_check;
       record_check(st, l, target);
+    }
+    if (signal) {
+      __threadfence_system();
+      *(volatile int *)signal = 1;
     }
   }
 }
@@ -490,9 +495,9 @@ long launch_l2_partial(const GridDims &g, const double *gf, const double *w2d, d
 }
 
 void launch_l2_finalize(const double *partial, long npart, double volume, SolverDeviceState *dst, int steps_per_check,
-                        double target, double *log10_out, hipStream_t st) {
+                        double target, double *log10_out, hipStream_t st, int *signal) {
   hipLaunchKernelGGL(l2_finalize_kernel, dim3(1), dim3(256), 0, st, partial, npart, volume, dst, steps_per_check,
-                     target, log10_out);
+                     target, log10_out, signal);
 }
 
 // ---------------------------------------------------------------------------------------
