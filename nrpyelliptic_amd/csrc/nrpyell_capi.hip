@@ -780,7 +780,7 @@ struct nrpyell_solver {
   double dt = 0.0;
   nrpyell_solve_options opt{};
   hipStream_t stream = nullptr;
-  int tx = 32, pl = 1, ntile0 = 0, ntile1 = 0;
+  int tx = 32, pl = 1, ntile0 = 0, ntile1 = 0, pair_rows = NRPYELL_PAIR_BC_ROWS;
   bool pair_path = false;  // FP64 steps as two launches of two substeps each
   int ybuf = 0;            // pair path: y_n currently in y_n_gfs (0) or k_even_gfs (1)
   double *coef64 = nullptr;   // metric coefficients (residual kernel)
@@ -855,7 +855,8 @@ struct nrpyell_solver {
     a.done = &dstate->done;
     a.tx = tx;
     a.pl = pl;
-    a.nbc_rows = (g.N1 + NRPYELL_BC_ROWS - 1) / NRPYELL_BC_ROWS;
+    a.bc_rows = NRPYELL_BC_ROWS;
+    a.nbc_rows = (g.N1 + a.bc_rows - 1) / a.bc_rows;
     a.ntile0 = ntile0;
     a.ntile1 = ntile1;
     a.i0_first = NRPYELL_NG + g.N0 - ntile0 * tx;
@@ -896,10 +897,11 @@ struct nrpyell_solver {
     a.out = ycur(1 - j);
     launch_substep_pair(a, 3, st, &order);
   }
-  // the pair kernel's BC blocks cover NRPYELL_PAIR_BC_ROWS rows each
+  // the pair kernel's BC blocks cover pair_rows rows each
   template <typename T>
   void pair_layout(SubstepArgs<T> &a) const {
-    a.nbc_rows = (g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS;
+    a.bc_rows = pair_rows;
+    a.nbc_rows = (g.N1 + a.bc_rows - 1) / a.bc_rows;
     a.nbc_mul = div_mul((unsigned)a.nbc_rows);
   }
   // RK4 steps in a graph: the pair path needs an even count (y_n back in y_n_gfs)
@@ -1080,7 +1082,7 @@ static void pair_block_order(nrpyell_solver *s) {
   s->order = BlockOrder{};
   if (!s->pair_path) return;
   const int ncu = cu_count();
-  const int nbc_rows = (s->g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS;
+  const int nbc_rows = (s->g.N1 + s->pair_rows - 1) / s->pair_rows;
   plan_block_order(ncu, nbc_rows * s->g.N2, s->ntile0, s->ntile1, s->g.N2 / s->pl, s->order);
 }
 
@@ -1160,6 +1162,20 @@ static bool four_planes_pay(long blocks, int ncu) {
 }
 static bool four_planes_pay_in_batch(long blocks, int ncu) { return 4 * blocks >= 5l * ncu; }
 
+// Rows per BC block of the two-substep kernel. On a grid whose blocks all run at once the step waits for
+// the BC blocks (64x64x4: 13.2 us per step, 10.1 without them, 12.8 without the interior blocks), whose
+// chain of dependent phases is shorter with 8 rows; on larger ones their halo rows' work counts. The
+// 32-wide kernels with one and two planes have both. us per RK4 step with 16 / 8 rows, by the number
+// of 8-row BC blocks and of all blocks: 16x16x6 13.1 / 11.7 (12, 24), 64x64x4 13.2 / 11.0 (32, 96), 64x64x16
+// 14.8 / 13.1 (128, 256), 96x64x8 14.0 / 11.3 (64, 160), 96x96x8 14.7 / 13.5 (96, 240), 128x64x16 18.0 / 15.6
+// (128, 384), 128x128x8 16.1 / 15.3 (128, 384); then 32x64x32 16.0 / 16.9 (256, 384), 96x96x16 18.7 / 19.1
+// (192, 480), 64x128x16 16.5 / 17.5 (256, 512), 128x128x16 19.8 / 22.2 (256, 768). Four rows gain nothing over 8.
+static int pair_bc_rows(const GridDims &g, int tx, int pl, long tiles, int ncu) {
+  const int R = NRPYELL_PAIR_BC_ROWS_SHORT;
+  const long bc = (long)g.N2 * ((g.N1 + R - 1) / R), all = tiles * (g.N2 / pl) + bc;
+  return tx == 32 && pl <= 2 && 2 * bc <= ncu && 2 * all <= 3l * ncu ? R : NRPYELL_PAIR_BC_ROWS;
+}
+
 // auto_planes: planes per thread where the caller's options leave them open; 0: chosen for this grid
 // alone on the GPU
 static int make_solver(griddata_struct *gd, REAL dt, const nrpyell_solve_options *opt, int auto_planes,
@@ -1228,6 +1244,8 @@ static int make_solver(griddata_struct *gd, REAL dt, const nrpyell_solve_options
     }
     s->tx = tx;
     s->pl = pl;
+    // (a batch's launches are shared by its members: 16 rows)
+    if (auto_planes == 0) s->pair_rows = pair_bc_rows(g, tx, pl, (long)s->ntile0 * s->ntile1, cu_count());
     {
       // two substeps per launch unless the caller asks for one: the BC blocks' reflected rows need
       // Nxx1 >= 10 (checked above), the phi windows work for any even Nxx2. Asking for two by number
@@ -1246,7 +1264,7 @@ static int make_solver(griddata_struct *gd, REAL dt, const nrpyell_solve_options
     }
     {
       // the kernels split block indices with div_by: exact while index x divisor <= 2^32
-      // (the two-substep kernel's BC blocks cover fewer rows: NRPYELL_PAIR_BC_ROWS >= 8)
+      // (BC blocks of the two-substep kernel: 8 rows or 16)
       const double lim = 4294967296.0, nbc = (double)((g.N1 + 7) / 8);
       const double nsub = (double)s->ntile0 * s->ntile1 * (g.N2 / pl);
       if (nsub * (g.N2 / pl) > lim || (double)s->ntile0 * s->ntile1 * s->ntile0 > lim || nbc * nbc * g.N2 > lim) {

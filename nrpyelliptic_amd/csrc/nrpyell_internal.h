@@ -43,11 +43,11 @@ struct SolverDeviceState {
 #ifndef NRPYELL_BC_ROWS
 #define NRPYELL_BC_ROWS (NRPYELL_BLOCK / 16)
 #endif
-// i1 rows per BC block of the two-substep kernel (each block also works on 10 halo rows; 8 and
-// 16 measured alike at 128x128x16 with 32x2 tiles, 16 faster with one-plane tiles)
-#ifndef NRPYELL_PAIR_BC_ROWS
+// i1 rows per BC block of the two-substep kernel. Each block also works on 10 halo rows, so fewer rows
+// are more work in all and a shorter chain per block: short ones where the chip has room for them
+// (nrpyell_capi.hip, pair_bc_rows).
 #define NRPYELL_PAIR_BC_ROWS 16
-#endif
+#define NRPYELL_PAIR_BC_ROWS_SHORT 8
 
 // Bookkeeping of one residual check (log10 L2 = l) taken after st->steps steps: history,
 // done = 1 at the target, 2 on NaN, 3 on divergence.
@@ -146,7 +146,8 @@ struct SubstepArgs {
   const int *done;  // nonzero: converged, every launch returns at once
   int tx;           // tile width along i0 (threads), tile height along i1 = blockDim/tx
   int pl;           // i2 planes per thread (1 or 2)
-  int nbc_rows;     // BC blocks per i2 plane: ceil(N1 / NRPYELL_BC_ROWS)
+  int bc_rows;      // rows per BC block
+  int nbc_rows;     // BC blocks per i2 plane: ceil(N1 / bc_rows)
   int ntile0, ntile1;
   int i0_first;     // two-substep kernel: i0 of the first tile's column 0 (tiles end at ilast)
   // div_mul of N2/pl, ntile0 and nbc_rows: the kernels split block indices by them

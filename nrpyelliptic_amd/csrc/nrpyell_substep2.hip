@@ -119,7 +119,7 @@ __device__ __forceinline__ int wrap2_arm(const GridDims &g, int j) {
 // Source row, source plane and i1 orientation of a row index that may lie beyond the grid's
 // stored ghost rows: the SinhSymTP reflection xx1 -> -xx1 (or 2 pi - xx1) with a half turn in phi.
 // Rows more than N1 - 10 beyond the last interior row occur only in the unused tail of a BC
-// block on a grid with N1 < NRPYELL_BC_ROWS + 10; they are clamped into the grid.
+// block on a grid with N1 < TYB + 10; they are clamped into the grid.
 __device__ __forceinline__ void vrow_source(const GridDims &g, int vr, int i2, int &row, int &pl, int &dir) {
   if (vr < NG) {
     row = min(2 * NG - 1 - vr, g.N1 + NG - 1);
@@ -146,8 +146,9 @@ constexpr int interior2_lds() {
   constexpr int NT = NRPYELL_BLOCK, TY = NT / TX, BOX = (TX + 2 * NG) * (TY + 2 * NG), NR = (BOX + NT - 1) / NT;
   return 2 * PL * NR * NT + 24 * TY + NRPYELL_FD_TABLE;
 }
+template <int TYB>
 constexpr int bc2_lds() {
-  constexpr int NT = NRPYELL_BLOCK, TYB = NRPYELL_PAIR_BC_ROWS, NR1 = TYB + 2 * NG;
+  constexpr int NT = NRPYELL_BLOCK, NR1 = TYB + 2 * NG;
   constexpr int NRB = ((TYB + 4 * NG) * 17 + NT - 1) / NT;
   return 2 * NRB * NT + NR1 * (24 + 10 + 24 + 2 + 12) + TYB * (10 + 30 + 8 + 10 + 2 + 12) + NRPYELL_FD_TABLE;
 }
@@ -382,8 +383,8 @@ __device__ __forceinline__ void interior2_body(const SubstepArgs<T> &a, const in
 // ---------------------------------------------------------------------------------------
 // Stage-s stencil point t of a BC block: (R1 row e, column col); t < 6 TYB: a tile row (e = NG
 // + t / 6) and a column ilast-6 .. ilast-1; then column ilast on R1 rows 0 .. TYB+2NG-1.
+template <int TYB>
 __device__ __forceinline__ void r1_stencil_point(int t, int ilast, int &e, int &col) {
-  constexpr int TYB = NRPYELL_PAIR_BC_ROWS;
   if (t < 6 * TYB) {
     e = NG + t / 6;
     col = ilast - 6 + t % 6;
@@ -393,15 +394,16 @@ __device__ __forceinline__ void r1_stencil_point(int t, int ilast, int &e, int &
   }
 }
 
-template <typename T, int PAIR, int MODE, bool HOME>
+template <typename T, int PAIR, int MODE, bool HOME, int TYB>
 __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, const int plane, T *lds) {
   constexpr int S0 = PAIR;
-  constexpr int NT = NRPYELL_BLOCK, TYB = NRPYELL_PAIR_BC_ROWS;
+  constexpr int NT = NRPYELL_BLOCK;
   constexpr int NVR = TYB + 4 * NG, NC = 17, NBOX = NVR * NC, NRB = (NBOX + NT - 1) / NT;
   // stage-s stencils: columns ilast-6 .. ilast-1 on the tile rows (the one-sided d_0 of stage
   // s+1's radiation terms reads them there only) and column ilast on every R1 row (d_1 there)
   constexpr int NR1 = TYB + 2 * NG, NI = 6 * TYB + NR1, NIR = (NI + NT - 1) / NT;
   constexpr int NA0 = NR1 * 12, NAR = (NA0 + NT - 1) / NT;  // stage-s radiation terms
+  constexpr int NIW = (NI + 63) / 64 * 64 % NT;             // threads of the waves that hold stencil points
   constexpr int NO0 = NR1 * 10, NOR = (NO0 + NT - 1) / NT;  // stage-s outer values
   constexpr int NGE = NR1 * 24, NGER = (NGE + NT - 1) / NT;  // geometry of the R1 rows
   constexpr int NARM = TYB * 30, NARMR = (NARM + NT - 1) / NT;  // i2 arms at (ilast, tile rows)
@@ -447,7 +449,7 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
 #pragma unroll
   for (int it = 0; it < NIR; it++) {
     int e, col;
-    r1_stencil_point(min(tid + NT * it, NI - 1), ilast, e, col);
+    r1_stencil_point<TYB>(min(tid + NT * it, NI - 1), ilast, e, col);
     int row, pl, dir;
     vrow_source(g, r0 - NG + e, i2, row, pl, dir);
     const unsigned k2 = (unsigned)row * s1s + col, p = (unsigned)pl * s2 + k2;
@@ -530,7 +532,7 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
     const int t = tid + NT * it;
     if (t < NI) {
       int e, col;
-      r1_stencil_point(t, ilast, e, col);
+      r1_stencil_point<TYB>(t, ilast, e, col);
       const int vr = r0 - NG + e;
       int row, pl, dir;
       vrow_source(g, vr, i2, row, pl, dir);
@@ -551,10 +553,12 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
       }
     }
   }
-  // ---- stage s's radiation terms A_pt (pt 0..5, both gridfunctions) on the R1 rows
+  // ---- stage s's radiation terms A_pt (pt 0..5, both gridfunctions) on the R1 rows, dealt out from
+  // the waves without a stencil point on: both are chains of FMAs, and the block's time on a small grid
+  // is the longest wave's (64x64x4 13.2 -> 12.5 us per step with 16 rows, 256x256x32 93.6 -> 92.9)
 #pragma unroll
   for (int it = 0; it < NAR; it++) {
-    const int t = tid + NT * it;
+    const int t = (tid + NT - NIW) % NT + NT * it;
     if (t < NA0) {
       const int e = t / 12, gf = (t % 12) / 6, pt = t % 6, vr = r0 - NG + e;
       int row, pl, dir;
@@ -645,9 +649,9 @@ __device__ __forceinline__ void bc2_body(const SubstepArgs<T> &a, const int rb, 
 // Blocks per CU: three, or two where a thread's four planes need more than 168 registers.
 constexpr int pair_occupancy(int pl) { return pl == 4 ? 2 : 3; }
 
-template <typename T, int PAIR, int TX, int PL, int MODE, bool HOME = false>
+template <typename T, int PAIR, int TX, int PL, int MODE, bool HOME = false, int TYB = NRPYELL_PAIR_BC_ROWS>
 __global__ void __launch_bounds__(NRPYELL_BLOCK, pair_occupancy(PL)) substep2_kernel(SubstepArgs<T> a, const BlockOrder ord) {
-  constexpr int NL = interior2_lds<TX, PL>() > bc2_lds() ? interior2_lds<TX, PL>() : bc2_lds();
+  constexpr int NL = interior2_lds<TX, PL>() > bc2_lds<TYB>() ? interior2_lds<TX, PL>() : bc2_lds<TYB>();
   __shared__ T lds[NL];
   __shared__ double s_red[NRPYELL_BLOCK / 64];
   const unsigned nb = (unsigned)(a.nbc_rows * a.g.N2), ni = gridDim.x - nb;
@@ -656,7 +660,7 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, pair_occupancy(PL)) substep2_ke
   const unsigned L = ordered ? v : blockIdx.x;
   if (L < nb) {
     const unsigned pln = div_by(L, a.nbc_mul);
-    bc2_body<T, PAIR, MODE, HOME>(a, (int)(L - pln * (unsigned)a.nbc_rows), (int)pln, lds);
+    bc2_body<T, PAIR, MODE, HOME, TYB>(a, (int)(L - pln * (unsigned)a.nbc_rows), (int)pln, lds);
     return;
   }
   const unsigned q = ordered ? L - nb : xcd_logical(L - nb, ni), ng = (unsigned)(a.g.N2 / PL);
@@ -673,7 +677,8 @@ template <int PAIR, int TX, int PL, int MODE>
 __global__ void __launch_bounds__(NRPYELL_BLOCK, pair_occupancy(PL))
     substep2_batched_kernel(const SubstepArgs<double> *__restrict__ cfgs, const int *__restrict__ block_cfg,
                             const int *__restrict__ block_first) {
-  constexpr int NL = interior2_lds<TX, PL>() > bc2_lds() ? interior2_lds<TX, PL>() : bc2_lds();
+  constexpr int TYB = NRPYELL_PAIR_BC_ROWS;
+  constexpr int NL = interior2_lds<TX, PL>() > bc2_lds<TYB>() ? interior2_lds<TX, PL>() : bc2_lds<TYB>();
   __shared__ double lds[NL];
   __shared__ double s_red[NRPYELL_BLOCK / 64];
   const unsigned q = xcd_logical(blockIdx.x, gridDim.x);
@@ -683,7 +688,7 @@ __global__ void __launch_bounds__(NRPYELL_BLOCK, pair_occupancy(PL))
   const unsigned local = q - block_first[c], nb = (unsigned)(a.nbc_rows * a.g.N2);
   if (local < nb) {
     const unsigned pln = div_by(local, a.nbc_mul);
-    bc2_body<double, PAIR, MODE, false>(a, (int)(local - pln * (unsigned)a.nbc_rows), (int)pln, lds);
+    bc2_body<double, PAIR, MODE, false, TYB>(a, (int)(local - pln * (unsigned)a.nbc_rows), (int)pln, lds);
     return;
   }
   const unsigned li = local - nb, ng = (unsigned)(a.g.N2 / PL);
@@ -740,6 +745,12 @@ void launch_substep_pair_batched(const SubstepArgs<double> *cfgs, const int *blo
 template <typename T, int PAIR, int MODE>
 static void launch_pair(const SubstepArgs<T> &a, hipStream_t st, const BlockOrder &o) {
   dim3 grd(a.nbc_rows * a.g.N2 + a.ntile0 * a.ntile1 * (a.g.N2 / a.pl)), blk(NRPYELL_BLOCK);
+  if (a.bc_rows == NRPYELL_PAIR_BC_ROWS_SHORT) {
+    constexpr int R = NRPYELL_PAIR_BC_ROWS_SHORT;
+    if (a.pl == 2) hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 2, MODE, false, R>), grd, blk, 0, st, a, o);
+    else hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 1, MODE, false, R>), grd, blk, 0, st, a, o);
+    return;
+  }
   if (a.pl == 4) {
     hipLaunchKernelGGL((substep2_kernel<T, PAIR, 32, 4, MODE>), grd, blk, 0, st, a, o);
     return;
@@ -768,31 +779,33 @@ void launch_substep_pair(const SubstepArgs<T> &a, int first_stage, hipStream_t s
 template void launch_substep_pair<double>(const SubstepArgs<double> &, int, hipStream_t, const BlockOrder *);
 template void launch_substep_pair<float>(const SubstepArgs<float> &, int, hipStream_t, const BlockOrder *);
 
-template <int PL, int MODE>
+template <int PL, int MODE, int TYB = NRPYELL_PAIR_BC_ROWS>
 static void step_in_place(SubstepArgs<double> &a, double *y_n, double *k_odd, double *copy, hipStream_t st,
                           const BlockOrder &o) {
   dim3 grd(a.nbc_rows * a.g.N2 + a.ntile0 * a.ntile1 * (a.g.N2 / PL)), blk(NRPYELL_BLOCK);
   a.in = a.yn = y_n;
   a.out = k_odd;
   a.copy = copy;
-  hipLaunchKernelGGL((substep2_kernel<double, 1, 32, PL, MODE, true>), grd, blk, 0, st, a, o);
+  hipLaunchKernelGGL((substep2_kernel<double, 1, 32, PL, MODE, true, TYB>), grd, blk, 0, st, a, o);
   a.in = k_odd;
   a.yn = copy;
   a.out = y_n;
-  hipLaunchKernelGGL((substep2_kernel<double, 3, 32, PL, MODE, true>), grd, blk, 0, st, a, o);
+  hipLaunchKernelGGL((substep2_kernel<double, 3, 32, PL, MODE, true, TYB>), grd, blk, 0, st, a, o);
 }
 
 void launch_step_in_place(SubstepArgs<double> a, double *y_n, double *k_odd, double *copy, hipStream_t st,
                           const BlockOrder *ord) {
   static const BlockOrder none{};
   const BlockOrder &o = ord ? *ord : none;
-  if (a.g.N2 >= 6) {
-    if (a.pl == 4) step_in_place<4, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
-    else if (a.pl == 2) step_in_place<2, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
-    else step_in_place<1, PAIR_RADIATION>(a, y_n, k_odd, copy, st, o);
-  } else {
-    if (a.pl == 4) step_in_place<4, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
-    else if (a.pl == 2) step_in_place<2, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
-    else step_in_place<1, PAIR_RADIATION_ANY>(a, y_n, k_odd, copy, st, o);
-  }
+  auto go = [&](auto mode) {
+    constexpr int M = decltype(mode)::value, R = NRPYELL_PAIR_BC_ROWS_SHORT;
+    const bool rows_short = a.bc_rows == R;
+    if (a.pl == 4) step_in_place<4, M>(a, y_n, k_odd, copy, st, o);
+    else if (a.pl == 2 && rows_short) step_in_place<2, M, R>(a, y_n, k_odd, copy, st, o);
+    else if (a.pl == 2) step_in_place<2, M>(a, y_n, k_odd, copy, st, o);
+    else if (rows_short) step_in_place<1, M, R>(a, y_n, k_odd, copy, st, o);
+    else step_in_place<1, M>(a, y_n, k_odd, copy, st, o);
+  };
+  if (a.g.N2 >= 6) go(IntC<PAIR_RADIATION>{});
+  else go(IntC<PAIR_RADIATION_ANY>{});
 }
