@@ -1235,7 +1235,7 @@ static int make_solver(griddata_struct *gd, REAL dt, const nrpyell_solve_options
     } else if (pl <= 0) {
       // Two planes per thread share the coefficients and most of the phi window; one plane leaves half
       // the work per block, which is faster while those blocks still get a CU each (us per RK4 step,
-      // one / two planes: 16x16x6 13.7 / 14.6, 64x64x4 13.3 / 13.6, 64x64x8 14.1 / 14.2; past that
+      // one / two planes, 16-row BC blocks: 16x16x6 13.7 / 14.6, 64x64x4 13.3 / 13.6, 64x64x8 14.1 / 14.2; past that
       // 64x64x16 16.8 / 15.1, 96x96x8 16.9 / 15.2, 128x128x16 23.5 / 20.2).
       const long blocks = (long)g.N2 * (s->ntile0 * s->ntile1 + (g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS);
       pl = tx >= 32 && blocks > cu_count() ? 2 : 1;

@@ -2,7 +2,7 @@
 // the resident solver, in FP64 and in the FP32 bulk phase of the mixed-precision solve (templated
 // on the arithmetic type T), with either outer BC on any even number of phi planes. Against four
 // one-substep launches per step: 128x128x16 20.2 / 26.3 us (radiation), 20.7 / 26.7 us (Sommerfeld),
-// 64x64x4 13.3 / 15.4 us.
+// 64x64x4 11.0 / 15.4 us.
 //
 // RK4 on  u_t = v - eta u,  v_t = c^2 (lap u + AA^2 / (8 (psi+u)^7))  couples neighbouring points
 // only through the stencil of u: the next stage's u is pointwise,
