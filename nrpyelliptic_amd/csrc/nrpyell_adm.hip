@@ -101,7 +101,7 @@ template <int ORDER>
 __global__ void __launch_bounds__(ADM_T) admbase_kernel(AdmArgs a) {
   constexpr int NP = ORDER + 1;
   __shared__ double s_w[3][NP][ADM_T];
-  __shared__ unsigned s_base[ADM_T];
+  __shared__ long s_base[ADM_T];  // the molecule's first point: a grid may have more than 2^32
   double *s_u = s_w[0][0];  // a point's sum replaces its first weight, which only its own lanes read
   const int tid = threadIdx.x;
   const long i = (long)blockIdx.x * ADM_T + tid;
@@ -132,8 +132,7 @@ __global__ void __launch_bounds__(ADM_T) admbase_kernel(AdmArgs a) {
       for (int m = 0; m < NP; m++) s_w[d][m][tid] = w[m];
     }
     if (!ok) a.err[1] = 1;
-    s_base[tid] =
-        ok ? (unsigned)f[0] + (unsigned)a.dims[0] * ((unsigned)f[1] + (unsigned)a.dims[1] * (unsigned)f[2]) : 0;
+    s_base[tid] = ok ? f[0] + a.dims[0] * (f[1] + a.dims[1] * (long)f[2]) : 0;
   }
   if (!ok) s_base[tid] = 0;  // such a point's sum is not used
   __syncthreads();
