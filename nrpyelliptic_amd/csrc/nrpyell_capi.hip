@@ -793,6 +793,8 @@ struct nrpyell_solver {
   double volume = 0.0;
   double *partial = nullptr;
   double *l2_out = nullptr;
+  const int *never_done = nullptr;  // stays 0 (behind l2_out)
+  bool run_on = false;              // launches ignore the done flag: timed steps are all taken
   SolverDeviceState *dstate = nullptr;
   SolverDeviceState *hstate = nullptr;  // pinned
   // FP32 shadow state
@@ -852,7 +854,7 @@ struct nrpyell_solver {
     a.cOB_v = (T)(c_fixed > 0 ? c_fixed : gd->params.vv_wavespeed_at_OB);
     a.eta = (T)gd->params.eta_damping;
     a.dt = (T)dt;
-    a.done = &dstate->done;
+    a.done = run_on ? never_done : &dstate->done;
     a.tx = tx;
     a.pl = pl;
     a.bc_rows = NRPYELL_BC_ROWS;
@@ -1299,7 +1301,9 @@ static int make_solver(griddata_struct *gd, REAL dt, const nrpyell_solve_options
     const long nblk_res = (long)((g.N0 + 63) / 64) * ((g.N1 + 3) / 4) * g.N2;
     const long nblk_sub = (long)s->ntile0 * s->ntile1 * (g.N2 / (pl < 2 ? pl : 2));
     s->partial = dalloc<double>(nblk_res > nblk_sub ? nblk_res : nblk_sub);
-    s->l2_out = dalloc<double>(1);
+    s->l2_out = dalloc<double>(2);
+    HIPCHK(hipMemsetAsync(s->l2_out, 0, 2 * sizeof(double), s->stream));
+    s->never_done = (const int *)(s->l2_out + 1);
     s->dstate = dalloc<SolverDeviceState>(1);
     HIPCHK(hipHostMalloc((void **)&s->hstate, sizeof(SolverDeviceState), hipHostMallocDefault));
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -1508,20 +1512,22 @@ extern "C" int nrpyell_solver_solve(nrpyell_solver *s, nrpyell_solve_result *res
 }
 
 // Exactly n RK4 steps of the production FP64 path (graph replay, stage-1 residual check every
-// step against an unreachable target so nothing stops early), bracketed by HIP events on the
+// step against an unreachable target, the launches on a flag that stays 0, so that a state that
+// diverges or becomes NaN does not stop them either), bracketed by HIP events on the
 // solver's stream. Returns the elapsed milliseconds and the final log10 L2.
 extern "C" int nrpyell_solver_timed_steps(nrpyell_solver *s, int n, double *ms_out, double *log10_out) {
   return api_call([&]() -> int {
-    const double keep = s->opt.log10_target;
-    s->opt.log10_target = -1e300;
     const int per = s->graph_steps64();
-    hipGraphExec_t g = capture(s, false, per, s->opt.log10_target);
-    s->opt.log10_target = keep;
-    hipGraphExec_t tail = nullptr;
-    if (n % per) {
-      s->opt.log10_target = -1e300;
-      tail = capture(s, false, n % per, s->opt.log10_target);
-      s->opt.log10_target = keep;
+    hipGraphExec_t g = nullptr, tail = nullptr;
+    {
+      struct Timed {
+        nrpyell_solver *s;
+        const double keep = s->opt.log10_target;
+        explicit Timed(nrpyell_solver *t) : s(t) { s->opt.log10_target = -1e300; s->run_on = true; }
+        ~Timed() { s->opt.log10_target = keep; s->run_on = false; }
+      } timed(s);
+      g = capture(s, false, per, s->opt.log10_target);
+      if (n % per) tail = capture(s, false, n % per, s->opt.log10_target);
     }
     reset_state(s);
     hipEvent_t e0, e1;
@@ -1592,6 +1598,7 @@ extern "C" int nrpyell_solver_time_substep(nrpyell_solver *s, int stage, int n, 
       }
       SubstepArgs<double> a = s->args<double>(1, f.y_n_gfs, f.k_odd_gfs, nullptr, f.y_nplus1_running_total_gfs,
                                               s->src64, s->kc64, s->geo64);
+      a.done = s->never_done;
       a.in = a.yn = f.y_n_gfs;
       a.out = f.k_odd_gfs;
       s->pair_layout(a);
@@ -1627,6 +1634,7 @@ extern "C" int nrpyell_solver_time_substep(nrpyell_solver *s, int stage, int n, 
     SubstepArgs<double> a =
         s->args<double>(stage, f.y_n_gfs, f.k_odd_gfs, f.k_even_gfs, f.y_nplus1_running_total_gfs, s->src64,
                         s->kc64, s->geo64);
+    a.done = s->never_done;  // every launch does the full work, whatever the fused check finds
     if (a.pl == 4) {  // the one-substep kernel has one and two planes
       a.pl = 2;
       a.ng_mul = div_mul((unsigned)(s->g.N2 / 2));
@@ -1635,7 +1643,7 @@ extern "C" int nrpyell_solver_time_substep(nrpyell_solver *s, int stage, int n, 
       a.l2_partial = s->partial;
       a.state = s->dstate;
       a.l2_volume = s->volume;
-      a.l2_target = -1e300;  // never "converges": every launch does the full work
+      a.l2_target = -1e300;
     }
     SubstepArgs<double> b = a;
     double *tmp = nullptr;
