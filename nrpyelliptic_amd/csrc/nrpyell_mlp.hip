@@ -34,16 +34,18 @@ struct MlpOffsets {
   long w[MLP_HIDDEN + 2], b[MLP_HIDDEN + 2];
 };
 
-// 1 / (1 + e^-z). The reciprocal is v_rcp_f32 (1 ulp) with one Newton step, and v_div_fixup_f32
-// restores the quotient's special values (1 / inf = 0, NaN): 4 instructions in the place of the
-// 10 of an FP32 division. Measured over 4 million z in [-30, 30], z * sigmoidf_(z) is the same
-// float as with the division (largest relative error against FP64 1.8e-6, from the exponential;
-// below z = -87.3, where the sigmoid is a denormal, it is 0).
+// 1 / (1 + e^-z). The reciprocal is v_rcp_f32 (1 ulp) with one Newton step: 4 instructions in the
+// place of the 10 of an FP32 division. It is taken of (1 + e^-z) / 4, and the Newton step brings the 4
+// back, because v_rcp_f32 gives 0 for a denormal reciprocal (z below -87.3); powers of two change no
+// other bit. Where e^-z is infinite the Newton step is NaN, which the clamp to [0, 1], an output modifier
+// of its last FMA, makes 0 (a NaN z stays NaN in z * sigmoidf_(z)).
+// Measured over 4 million z in [-100, 30]: z * sigmoidf_(z) is the same float as with the division for z
+// above -30; below, 0.4 % differ in a denormal's last bit, at the same error against FP64 (rms 1.6e-6,
+// largest 4.1e-6, from the exponential).
 __device__ __forceinline__ float sigmoidf_(float z) {
-  const float d = 1.0f + __expf(-z);
-  float r = __builtin_amdgcn_rcpf(d);
-  r = fmaf(fmaf(-d, r, 1.0f), r, r);
-  return __builtin_amdgcn_div_fixupf(r, d, 1.0f);
+  const float d = fmaf(0.25f, __expf(-z), 0.25f);
+  const float r = __builtin_amdgcn_rcpf(d), q = 0.25f * r;
+  return __builtin_amdgcn_fmed3f(fmaf(fmaf(-d, r, 1.0f), q, q), 0.0f, 1.0f);
 }
 __device__ __forceinline__ bf16_t to_bf16(float x) { return (bf16_t)x; }
 
@@ -558,8 +560,8 @@ __global__ void mlp_adam_kernel(long n, const float *__restrict__ g, AdamArgs o)
 // and load, FI_PF inner steps ahead of their use and across the layer boundary. The kernel is
 // bound by the activations' vector instructions (1280 per row, each an exponential, a reciprocal
 // and about 8 more; the MFMAs need 58 us of the 186 at 2.5 PFLOP/s) and overlaps them with other
-// waves' MFMAs: four blocks per CU, which the single buffer (40 KB of LDS) and 124 registers per
-// lane allow. 262 144 rows: 186 us, 786 TFLOP/s (two ping-pong buffers, row-major weights loaded
+// waves' MFMAs: four blocks per CU, which the single buffer (40 KB of LDS) and 125 registers per
+// lane allow (one body for all five layers takes 160: layer 1 stands by itself). 262 144 rows: 186 us, 786 TFLOP/s (two ping-pong buffers, row-major weights loaded
 // where they are used and FP32 divisions: 390 us, 375 TFLOP/s; the same outputs).
 constexpr int FI_R = 64, FI_LD = MLP_W + 8;  // rows per block; LDS row stride (528 B)
 constexpr int FI_PF = 4;                     // inner steps of weights in flight
@@ -593,7 +595,7 @@ __device__ __forceinline__ void fi_layer(const bf16_t *H, const bf16_t *__restri
   }
 }
 
-__global__ void __launch_bounds__(256, 3) mlp_forward_fused_kernel(const bf16_t *__restrict__ X,
+__global__ void __launch_bounds__(256, 4) mlp_forward_fused_kernel(const bf16_t *__restrict__ X,
                                                                    const bf16_t *__restrict__ pws,
                                                                    const float *__restrict__ p, MlpOffsets off,
                                                                    WeightCopies wc, long M, float *__restrict__ y) {
@@ -620,12 +622,8 @@ __global__ void __launch_bounds__(256, 3) mlp_forward_fused_kernel(const bf16_t 
   for (int l = 0; l < MLP_HIDDEN; l++) s_b[l][tid] = p[off.b[l + 1] + tid];
   __syncthreads();
   const bf16_t *H = Hbuf + li * FI_LD + 8 * lj;
-  for (int l = 1; l <= MLP_HIDDEN; l++) {
-    floatx16 acc[2][2];
-    if (l == 1)
-      fi_layer<MLP_K0>(H, W, wv, acc);
-    else
-      fi_layer<MLP_W>(H, W, wv, acc);
+  // the activations of layer l from its accumulators, between the layer's products and the next one's
+  auto activate = [&](int l, const floatx16 (&acc)[2][2]) {
     if (l < MLP_HIDDEN) {  // the next layer's first weights, in flight during the activations
       W = pws + wc.fs[l + 1] + (long)(2 * wave) * (MLP_W / 16) * 512 + 8 * lane;
 #pragma unroll
@@ -654,6 +652,14 @@ __global__ void __launch_bounds__(256, 3) mlp_forward_fused_kernel(const bf16_t 
         }
       }
     __syncthreads();
+  };
+  floatx16 z[2][2];
+  fi_layer<MLP_K0>(H, W, wv, z);
+  activate(1, z);
+#pragma unroll 1
+  for (int l = 2; l <= MLP_HIDDEN; l++) {
+    fi_layer<MLP_W>(H, W, wv, z);
+    activate(l, z);
   }
   // output layer: wave w sums columns 64w..64w+63 of every row, then the 4 partials are added
   const float *wout = p + off.w[MLP_HIDDEN + 1] + 64 * wave;
