@@ -352,6 +352,8 @@ int nrpyell_solver_timed_steps(nrpyell_solver *s, int n, double *ms, double *log
 int nrpyell_set_eta_damping(griddata_struct *gd, double eta);
 /* RK4 substeps per launch of the solver's FP64 steps (1 or 2, see substeps_per_launch). */
 int nrpyell_solver_substeps_per_launch(nrpyell_solver *s);
+/* i2 planes per thread of the solver's kernels, as asked for or as chosen (see planes); 0 for a null solver. */
+int nrpyell_solver_planes(const nrpyell_solver *s);
 /* Residual history of the last solve: (steps completed, log10 L2) pairs; returns the count. */
 int nrpyell_solver_history(nrpyell_solver *s, int max, int *steps, double *log10_l2);
 /* Block placement of the solver's two-substep kernel: out[L] (L < max) = the block that the
@@ -377,6 +379,8 @@ int nrpyell_batch_create(griddata_struct **griddatas, const double *dts, const i
                          int n, const nrpyell_solve_options *opt, nrpyell_batch **out);
 /* Relax every configuration to opt->log10_target; res has n entries. */
 int nrpyell_batch_solve(nrpyell_batch *b, nrpyell_solve_result *res, double *seconds);
+/* nrpyell_solver_planes of member k; 0 for a null batch or no such member. */
+int nrpyell_batch_planes(const nrpyell_batch *b, int k);
 int nrpyell_batch_destroy(nrpyell_batch *b);
 
 /* Learned initial guess: coordinate MLP (64 padded input features -> 5 x [Linear 256 + SiLU]

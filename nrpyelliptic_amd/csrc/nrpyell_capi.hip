@@ -1153,16 +1153,29 @@ extern "C" void nrpyell_default_options(nrpyell_solve_options *o) {
 // make one full round of two per CU or many rounds. us per RK4 step, two / four planes, by four-plane
 // blocks: 256 (128x128x16) 20.8 / 22.3, 320 (160x128x16) 22.5 / 24.5, 476 (200x130x16) 33.0 / 32.0, 512
 // (256x128x16) 34.6 / 31.5, 640 (256x160x16) 40.6 / 41.4, 800 (160x160x32) 51.4 / 51.5, 1024 (256x256x16)
-// 56.5 / 52.4, 2048 (256x256x32) 101.2 / 96.1, 4096 (512x256x32) 240 / 212. In a batch the BC blocks and
-// the members' ragged tiles fill the gaps: 2 members (328 blocks) 32.4 / 31.2, 8 (1488) 87.2 / 81.0,
-// 16 (2980) 178 / 155, 48 661 / 574.
+// 56.5 / 52.4, 2048 (256x256x32) 101.2 / 96.1, 4096 (512x256x32) 240 / 212.
+// In a batch the blocks of the members follow each other without a placement, BC blocks among them, and
+// members on other planes are launches of their own. Four planes pay where the BC blocks are few and the
+// launch has many blocks; very many (15 per CU) also for the Sommerfeld BC, whose BC blocks cost more, and
+// beside such other launches. us per step, two / four planes, by four-plane and BC blocks of the batch:
+// radiation 618 and 336 46.5 / 44.6, 928 and 480 61.8 / 60.3, 1336 and 328 69.9 / 65.3, 1638 and 1136 101.4 / 95.7,
+// 2656 and 1344 178 / 155, 5046 and 2512 363 / 328; fewer blocks: 560 and 232 42.0 / 44.3, 294 and 168 27.0 / 28.7;
+// more BC blocks: 1520 and 1344 99.8 / 102.6, 420 and 432 38.9 / 43.7, 484 and 1024 54.3 / 63.2; beside members with 6
+// planes: 924 and 452 67.6 / 73.4, 1922 and 1120 154.6 / 138.0, 2396 and 1152 147.2 / 149.3, 3068 and 1520 215 / 202.
+// Sommerfeld: 1336 and 328 69.8 / 70.3, 2142 and 1336 126.2 / 137.2, 2728 and 1432 169.5 / 165.5, 5046 and 2512 361 / 342.
 static bool four_planes_allowed(const GridDims &g, int tx, const nrpyell_solve_options &o) {
   return tx == 32 && g.N2 % 4 == 0 && o.substeps_per_launch != 1;
 }
 static bool four_planes_pay(long blocks, int ncu) {
   return 4 * blocks >= 15l * ncu || (4 * blocks >= 7l * ncu && blocks <= 2l * ncu);
 }
-static bool four_planes_pay_in_batch(long blocks, int ncu) { return 4 * blocks >= 5l * ncu; }
+// all_radiation: the radiation BC, and no member on other planes
+static bool four_planes_pay_in_batch(long blocks, long bc_blocks, bool all_radiation, int ncu) {
+  const long all = blocks + bc_blocks;
+  if (4 * bc_blocks > 3 * blocks) return false;
+  if (all >= 15l * ncu) return true;
+  return all_radiation && (all >= 8l * ncu || (2 * all >= 7l * ncu && 5 * bc_blocks <= 3 * blocks));
+}
 
 // Rows per BC block of the two-substep kernel. On a grid whose blocks all run at once the step waits for
 // the BC blocks (64x64x4: 13.2 us per step, 10.1 without them, 12.8 without the interior blocks), whose
@@ -1569,6 +1582,8 @@ extern "C" int nrpyell_set_eta_damping(griddata_struct *gd, double eta) {
 
 extern "C" int nrpyell_solver_substeps_per_launch(nrpyell_solver *s) { return s ? (s->pair_path ? 2 : 1) : 0; }
 
+extern "C" int nrpyell_solver_planes(const nrpyell_solver *s) { return s ? s->pl : 0; }
+
 extern "C" int nrpyell_solver_history(nrpyell_solver *s, int max, int *steps, double *log10_l2) {
   return api_call([&]() -> int {
     read_state(s);
@@ -1929,13 +1944,19 @@ extern "C" int nrpyell_batch_create(griddata_struct **gds, const double *dts, co
       const nrpyell_solve_options o = options_of(k);
       return o.planes <= 0 && four_planes_allowed(dims_from_params(&gds[k]->params), o.tile_i0 > 0 ? o.tile_i0 : 32, o);
     };
-    long blocks4 = 0;
+    long blocks4 = 0, bc_blocks = 0;
+    bool all_radiation = b->opt.outer_bc == NRPYELL_OUTER_BC_RADIATION;
     for (int k = 0; k < n; k++) {
       const GridDims g = dims_from_params(&gds[k]->params);
       const int ty = NRPYELL_BLOCK / 32;
-      if (four(k)) blocks4 += (long)((g.N0 + 31) / 32) * ((g.N1 + ty - 1) / ty) * (g.N2 / 4);
+      if (four(k)) {
+        blocks4 += (long)((g.N0 + 31) / 32) * ((g.N1 + ty - 1) / ty) * (g.N2 / 4);
+        bc_blocks += (long)((g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS) * g.N2;
+      } else {
+        all_radiation = false;
+      }
     }
-    const bool pay = four_planes_pay_in_batch(blocks4, cu_count());
+    const bool pay = four_planes_pay_in_batch(blocks4, bc_blocks, all_radiation, cu_count());
     for (int k = 0; k < n; k++) {
       const nrpyell_solve_options o = options_of(k);
       nrpyell_solver *s = nullptr;
@@ -2055,6 +2076,10 @@ extern "C" int nrpyell_batch_solve(nrpyell_batch *b, nrpyell_solve_result *res, 
     if (rc == NRPYELL_ENOTCONVERGED) set_last_error("some configurations diverged or reached max_steps");
     return rc;
   });
+}
+
+extern "C" int nrpyell_batch_planes(const nrpyell_batch *b, int k) {
+  return b && k >= 0 && k < (int)b->solvers.size() ? b->solvers[k]->pl : 0;
 }
 
 extern "C" int nrpyell_batch_destroy(nrpyell_batch *b) {

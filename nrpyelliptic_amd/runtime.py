@@ -102,6 +102,8 @@ def lib() -> C.CDLL:
     L.nrpyell_solver_timed_steps.argtypes = [vp, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_double)]
     L.nrpyell_solver_history.argtypes = [vp, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_double)]
     L.nrpyell_solver_substeps_per_launch.argtypes = [vp]
+    L.nrpyell_solver_planes.argtypes = [vp]
+    L.nrpyell_batch_planes.argtypes = [vp, C.c_int]
     L.nrpyell_solver_block_order.argtypes = [vp, C.POINTER(C.c_ushort), C.c_int]
     L.nrpyell_block_order_plan.argtypes = [C.c_int] * 6 + [C.POINTER(C.c_ushort), C.c_int]
     L.nrpyell_set_eta_damping.argtypes = [C.POINTER(abi.griddata_struct), C.c_double]
@@ -512,6 +514,11 @@ class Solver:
         """1 or 2: RK4 substeps per launch of the FP64 steps."""
         return lib().nrpyell_solver_substeps_per_launch(self.h)
 
+    @property
+    def planes(self) -> int:
+        """phi planes per thread of the kernels, as asked for or as chosen."""
+        return lib().nrpyell_solver_planes(self.h)
+
     def block_order(self) -> np.ndarray:
         """Placement of the two-substep kernel's blocks: entry L is the block (BC blocks first,
         then interior blocks in tile order) that workgroup L of a launch computes; empty when the
@@ -554,6 +561,11 @@ class BatchSolver:
         pl = (C.c_int * n)(*[int(t[1]) for t in pairs])
         self.h = C.c_void_p()
         check(lib().nrpyell_batch_create(gds, dts, tl, pl, n, C.byref(self.opts), C.byref(self.h)), "batch_create")
+
+    @property
+    def planes(self) -> list:
+        """Each member's Solver.planes."""
+        return [lib().nrpyell_batch_planes(self.h, k) for k in range(len(self.problems))]
 
     def solve(self):
         n = len(self.problems)
