@@ -1149,11 +1149,21 @@ extern "C" void nrpyell_default_options(nrpyell_solve_options *o) {
 // Four planes per thread (two-substep kernel, 32-wide tiles): the window of planes per thread is 14
 // for 4 points instead of 12 for 2, a quarter fewer vector loads, whose rate bounds the kernel once
 // many blocks hide its latencies (texture data unit 66 / 76 % busy at 256x256x32); but it takes 168 / 241
-// registers, so two of its blocks fit a CU where three of the others do. It pays where the blocks
-// make one full round of two per CU or many rounds. us per RK4 step, two / four planes, by four-plane
-// blocks: 256 (128x128x16) 20.8 / 22.3, 320 (160x128x16) 22.5 / 24.5, 476 (200x130x16) 33.0 / 32.0, 512
-// (256x128x16) 34.6 / 31.5, 640 (256x160x16) 40.6 / 41.4, 800 (160x160x32) 51.4 / 51.5, 1024 (256x256x16)
-// 56.5 / 52.4, 2048 (256x256x32) 101.2 / 96.1, 4096 (512x256x32) 240 / 212.
+// registers, so two of its blocks fit a CU where three of the others do. For a grid alone it pays in
+// these ranges (four-plane blocks; BC blocks; us per RK4 step with two / four planes, FP64):
+// - 1.75 to 2 blocks per CU: with the BC blocks no more than three per CU (448; 224 128x224x16 33.9 / 30.8, 480; 192
+//   160x188x16 33.0 / 29.9, 512; 128 253x128x16 33.1 / 29.9), or with them two full rounds (512; 512 61x256x32 41.4 / 39.8);
+//   not between (480; 320 96x160x32 38.8 / 39.8, 448; 448 53x218x32 39.5 / 39.7) and not beyond (512; 1024 32x256x64
+//   49.8 / 52.0). In FP32 the two-plane kernel is better still with few blocks (448; 112 253x108x16 two / four 0.98).
+// - 4.5 per CU and more: BC blocks at most three quarters of them (1200; 416 179x198x32 64.7 / 63.3, 1600; 640 160x316x32
+//   82.0 / 78.0, 2048; 512 256x256x32 100.7 / 93.2, 4096; 512 512x256x32 239 / 213; but 1024; 2048 32x256x128 87.0 / 89.1)
+// - 3.75 to 4.5, FP64: the same (960; 240 256x160x24 53.4 / 50.2, 1024; 256 256x256x16 53.9 / 50.1, 1104; 384 192x178x32
+//   61.4 / 57.1, 1024; 512 123x256x32 58.9 / 56.7, 1008; 672 96x222x48 63.8 / 61.5) but for BC blocks between three
+//   eighths and four ninths of them, which is five tiles across (960; 384 160x90x64 55.9 / 58.7, 1120; 448
+//   160x112x64 67.5 / 69.6, 1140; 480 160x152x48 65.5 / 67.3). In FP32 0.96 to 1.03, no gain in the mean.
+// Elsewhere two planes are as good or better: 256 (128x128x16) 20.8 / 22.3, 640; 160 253x160x16 38.4 / 39.8, 648; 448
+// 85x210x32 44.6 / 46.7. The Sommerfeld BC gains the same or a few per cent less. Over 160 grids the rule's choice of four
+// planes is 3.4 % faster than two in the mean, 2.4 % slower at worst (320x72x48).
 // In a batch the blocks of the members follow each other without a placement, BC blocks among them, and
 // members on other planes are launches of their own. Four planes pay where the BC blocks are few and the
 // launch has many blocks; very many (15 per CU) also for the Sommerfeld BC, whose BC blocks cost more, and
@@ -1166,8 +1176,13 @@ extern "C" void nrpyell_default_options(nrpyell_solve_options *o) {
 static bool four_planes_allowed(const GridDims &g, int tx, const nrpyell_solve_options &o) {
   return tx == 32 && g.N2 % 4 == 0 && o.substeps_per_launch != 1;
 }
-static bool four_planes_pay(long blocks, int ncu) {
-  return 4 * blocks >= 15l * ncu || (4 * blocks >= 7l * ncu && blocks <= 2l * ncu);
+static bool four_planes_pay(long blocks, long bc_blocks, bool fp32, int ncu) {
+  const long all = blocks + bc_blocks;
+  if (2 * blocks >= 9l * ncu) return 4 * bc_blocks <= 3 * blocks;
+  if (4 * blocks >= 15l * ncu)
+    return !fp32 && 4 * bc_blocks <= 3 * blocks && (8 * bc_blocks <= 3 * blocks || 9 * bc_blocks >= 4 * blocks);
+  if (4 * blocks < 7l * ncu || blocks > 2l * ncu || (fp32 && 4 * all < 9l * ncu)) return false;
+  return all <= 3l * ncu || (8 * all > 31l * ncu && all <= 4l * ncu);
 }
 // all_radiation: the radiation BC, and no member on other planes
 static bool four_planes_pay_in_batch(long blocks, long bc_blocks, bool all_radiation, int ncu) {
@@ -1252,9 +1267,11 @@ static int make_solver(griddata_struct *gd, REAL dt, const nrpyell_solve_options
       // the work per block, which is faster while those blocks still get a CU each (us per RK4 step,
       // one / two planes, 16-row BC blocks: 16x16x6 13.7 / 14.6, 64x64x4 13.3 / 13.6, 64x64x8 14.1 / 14.2; past that
       // 64x64x16 16.8 / 15.1, 96x96x8 16.9 / 15.2, 128x128x16 23.5 / 20.2).
-      const long blocks = (long)g.N2 * (s->ntile0 * s->ntile1 + (g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS);
-      pl = tx >= 32 && blocks > cu_count() ? 2 : 1;
-      if (four_planes_allowed(g, tx, s->opt) && four_planes_pay((long)s->ntile0 * s->ntile1 * (g.N2 / 4), cu_count()))
+      const long tiles = (long)s->ntile0 * s->ntile1,
+                 bc_blocks = (long)g.N2 * ((g.N1 + NRPYELL_PAIR_BC_ROWS - 1) / NRPYELL_PAIR_BC_ROWS);
+      pl = tx >= 32 && g.N2 * tiles + bc_blocks > cu_count() ? 2 : 1;
+      if (four_planes_allowed(g, tx, s->opt) &&
+          four_planes_pay(tiles * (g.N2 / 4), bc_blocks, s->opt.precision == 32, cu_count()))
         pl = 4;
     }
     s->tx = tx;
