@@ -10,7 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
-#include <mutex>
+#include <memory>
 #include <string>
 
 #include "nrpyell_common.h"
@@ -199,19 +199,6 @@ __global__ void __launch_bounds__(ADM_T) admbase_kernel(AdmArgs a) {
   for (int c = 0; c < NRPYELL_ADM_NOUT; c++) __builtin_nontemporal_store(v[c], a.out[c] + i);
 }
 
-// The two error flags of a call: pinned host memory that the kernel writes and the host reads after
-// it, without an allocation, a clearing or a copy per call. One pair for the process (portable: any
-// device writes it), held with the lock from clearing to reading.
-std::mutex g_err_mu;
-struct ErrFlags {
-  int *host = nullptr, *dev = nullptr;
-  ErrFlags() {
-    HIPCHK(hipHostMalloc((void **)&host, 2 * sizeof(int),
-                         hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
-    HIPCHK(hipHostGetDevicePointer((void **)&dev, host, 0));
-  }
-};
-
 }  // namespace
 
 // Drop-in for NRPyEllipticET_conformally_flat_BBH_Initialize_ADMBase (Cactus types replaced by
@@ -298,11 +285,17 @@ extern "C" int nrpyell_Initialize_ADMBase(const griddata_struct *gd, const nrpye
     for (int c = 0; c < NRPYELL_ADM_NOUT; c++) a.out[c] = outs[c];
     a.n = n;
     a.sinh_1w = sinh(1.0 / p->SINHWAA);
-    std::lock_guard<std::mutex> lk(g_err_mu);
-    static ErrFlags flags;
-    volatile int *err = flags.host;
-    err[0] = err[1] = 0;
+    // The call's two error flags: pinned host memory that the kernel writes and the host reads after it,
+    // without an allocation, a clearing or a copy. In device memory where the pool has none left.
+    PinnedLine flags;
+    std::unique_ptr<DevBuf<int>> dev_flags;
+    int err[2] = {0, 0};
     a.err = flags.dev;
+    if (!flags.dev) {
+      dev_flags = std::make_unique<DevBuf<int>>(2);
+      a.err = dev_flags->p;
+      HIPCHK(hipMemset(a.err, 0, sizeof(err)));
+    }
     const dim3 grd((unsigned)((n + ADM_T - 1) / ADM_T)), blk(ADM_T);
     switch (opt->interpolation_order) {
       case 1: hipLaunchKernelGGL(admbase_kernel<1>, grd, blk, 0, 0, a); break;
@@ -314,6 +307,12 @@ extern "C" int nrpyell_Initialize_ADMBase(const griddata_struct *gd, const nrpye
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(0));
+    if (dev_flags) {
+      HIPCHK(hipMemcpy(err, a.err, sizeof(err), hipMemcpyDeviceToHost));
+    } else {
+      for (int k = 0; k < 2; k++) err[k] = ((volatile int *)flags.host)[k];
+      flags.give_back();
+    }
     if (err[1] == 0 && err[0] != 0) {
       set_last_error("NAN found in (xx0,xx1,xx2) after moving the point by NRPy_epsilon; consider increasing "
                      "NRPy_epsilon");

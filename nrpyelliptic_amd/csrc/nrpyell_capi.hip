@@ -107,14 +107,13 @@ __global__ void signal_kernel(int *flag) {
   *(volatile int *)flag = 1;
 }
 namespace {
-// The flags of concurrent calls: one page of pinned memory (portable: any device writes it), a cache line
-// each, one per call in flight.
-struct WaitFlags {
+// The lines of concurrent calls: one page (portable: any device writes it), one line per call in flight.
+struct LinePool {
   static constexpr int N = 64, STRIDE = 16;
   std::mutex mu;
   int *host = nullptr, *dev = nullptr;
   std::vector<int> unused;
-  ~WaitFlags() {
+  ~LinePool() {
     if ((int)unused.size() == N) (void)hipHostFree(host);
   }
   int take() {
@@ -138,24 +137,32 @@ struct WaitFlags {
     unused.push_back(k);
   }
 };
-WaitFlags g_wait_flags;
+LinePool g_lines;
+}  // namespace
 
-// One wait: take a flag, launch what sets it, wait. Without a free flag (64 calls in flight) it waits the
-// ordinary way. A flag is not handed out again when the stream failed, as its kernel may still write it.
+PinnedLine::PinnedLine() {
+  const int k = g_lines.take();
+  if (k < 0) return;
+  host = g_lines.host + k;
+  dev = g_lines.dev + k;
+  for (int i = 0; i < LinePool::STRIDE; i++) ((volatile int *)host)[i] = 0;
+}
+void PinnedLine::give_back() {
+  if (host) g_lines.give((int)(host - g_lines.host));
+  host = dev = nullptr;
+}
+
+namespace {
+// One wait: take a flag, launch what sets it, wait. Without a free flag it waits the ordinary way.
 class StreamWait {
  public:
-  StreamWait() : k_(g_wait_flags.take()) {
-    if (k_ >= 0) *(volatile int *)(g_wait_flags.host + k_) = 0;
-  }
-  StreamWait(const StreamWait &) = delete;
-  StreamWait &operator=(const StreamWait &) = delete;
-  int *flag() const { return k_ >= 0 ? g_wait_flags.dev + k_ : nullptr; }
+  int *flag() const { return line_.dev; }
   void signal(hipStream_t st) {
-    if (k_ >= 0) hipLaunchKernelGGL(signal_kernel, dim3(1), dim3(1), 0, st, flag());
+    if (line_.dev) hipLaunchKernelGGL(signal_kernel, dim3(1), dim3(1), 0, st, line_.dev);
   }
   void wait(hipStream_t st) {
     HIPCHK(hipGetLastError());
-    const volatile int *f = k_ >= 0 ? g_wait_flags.host + k_ : nullptr;
+    const volatile int *f = line_.host;
     const auto t0 = std::chrono::steady_clock::now();
     for (int n = 1; !f || *f == 0; n++)
       if (!f || (n % 64 == 0 && std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() >
@@ -164,11 +171,11 @@ class StreamWait {
         break;
       }
     std::atomic_thread_fence(std::memory_order_acquire);
-    if (k_ >= 0) g_wait_flags.give(k_);
+    line_.give_back();
   }
 
  private:
-  int k_;
+  PinnedLine line_;
 };
 }  // namespace
 

@@ -282,6 +282,17 @@ struct DevBuf {
   DevBuf &operator=(const DevBuf &) = delete;
 };
 
+// A cache line of pinned host memory for flags that a call's kernels write and the host reads (16 ints), from
+// a bounded pool of the process; nullptr where the pool has none left (64 calls in flight). It goes back
+// with give_back() once no kernel can write it any more; a call that fails on the GPU keeps it.
+struct PinnedLine {
+  int *host = nullptr, *dev = nullptr;
+  PinnedLine();
+  void give_back();
+  PinnedLine(const PinnedLine &) = delete;
+  PinnedLine &operator=(const PinnedLine &) = delete;
+};
+
 template <typename F>
 int api_call(F &&f) noexcept {
   try {
