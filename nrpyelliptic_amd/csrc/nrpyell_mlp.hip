@@ -883,7 +883,8 @@ struct nrpyell_mlp {
   hipStream_t st = nullptr;
   ~nrpyell_mlp() {
     (void)hipFree(params);
-    release_seed();
+    release_seed_rows();
+    release_seed_xx();
     release();
     if (st) (void)hipStreamDestroy(st);
   }
@@ -904,23 +905,32 @@ struct nrpyell_mlp {
     ws = nullptr;
     cap = 0;
   }
-  void release_seed() {
+  void release_seed_rows() {
     (void)hipFree(seedX); (void)hipFree(seed_scale); (void)hipFree(seed_idx); (void)hipFree(seed_y);
-    (void)hipFree(seed_xx);
-    seedX = nullptr; seed_scale = nullptr; seed_idx = nullptr; seed_y = nullptr; seed_xx = nullptr;
+    seedX = nullptr; seed_scale = nullptr; seed_idx = nullptr; seed_y = nullptr;
     seed_cap = 0;
+  }
+  void release_seed_xx() {
+    (void)hipFree(seed_xx);
+    seed_xx = nullptr;
     seed_nxx = 0;
   }
+  // The rows' arrays and the coordinates' grow apart: a grid with more of one and fewer of the other takes
+  // nothing away from the next. A failed allocation leaves the size 0: the next seed allocates again.
   void ensure_seed(long rows, int nxx) {
-    if (rows <= seed_cap && nxx <= seed_nxx) return;
-    release_seed();  // a failed allocation below leaves seed_cap 0: the next seed allocates again
-    seed_xx = mlp_alloc<double>((size_t)nxx);
-    seed_nxx = nxx;
-    seedX = mlp_alloc<bf16_t>((size_t)rows * MLP_K0);
-    seed_scale = mlp_alloc<double>((size_t)rows);
-    seed_idx = mlp_alloc<long>((size_t)rows);
-    seed_y = mlp_alloc<float>((size_t)rows);
-    seed_cap = rows;
+    if (rows > seed_cap) {
+      release_seed_rows();
+      seedX = mlp_alloc<bf16_t>((size_t)rows * MLP_K0);
+      seed_scale = mlp_alloc<double>((size_t)rows);
+      seed_idx = mlp_alloc<long>((size_t)rows);
+      seed_y = mlp_alloc<float>((size_t)rows);
+      seed_cap = rows;
+    }
+    if (nxx > seed_nxx) {
+      release_seed_xx();
+      seed_xx = mlp_alloc<double>((size_t)nxx);
+      seed_nxx = nxx;
+    }
   }
   void ensure(int M) {
     if (M <= cap) return;
