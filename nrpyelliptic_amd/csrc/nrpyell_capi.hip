@@ -1018,7 +1018,11 @@ static void plan_block_order(int ncu, int nb, int ntile0, int ntile1, int ng, Bl
   order = BlockOrder{};
   const int ni = ntile0 * ntile1 * ng, n = nb + ni;
   const int P = ncu / 8;
-  // one round of resident blocks (3 per CU: __launch_bounds__(256, 3), 37 KB of LDS each)
+  // One round of resident blocks: 3 per CU (__launch_bounds__(256, 3), 37 KB of LDS each). With four planes
+  // per thread a CU holds two, and the third starts where one of them ends; the placement gains there
+  // too (us per RK4 step, kernel's own order / placed: 128x224x16, 672 blocks, 32.6 / 30.8; 253x128x16, 640 blocks,
+  // 31.6 / 29.9; 192x80x32, 640 blocks, 33.4 / 32.5; 128x256x16, 768 blocks, 33.2 / 33.0), but for 768 blocks on
+  // 64 phi planes (128x64x64 36.0 / 37.3).
   if (ncu % 8 != 0 || P <= 0 || n > NRPYELL_ORDER_MAX || n > 3 * ncu || nb % 8 || ni % 8) return;
   const int per = ni / 8, nx = n / 8;
   struct Item {

@@ -82,3 +82,20 @@ def test_few_planes(grid, bc):
             assert np.array_equal(got, P.get("y_n_gfs"))
     finally:
         P.close()
+
+
+@pytest.mark.parametrize("grid,bc_blocks,blocks", [((256, 128, 16), 128, 640), ((128, 256, 16), 256, 768),
+                                                   ((256, 256, 32), 512, 0)])
+def test_placement_with_four_planes(grid, bc_blocks, blocks):
+    """Placed like the other kernels up to three blocks per CU: a permutation, the BC blocks first."""
+    P = problem(grid)
+    try:
+        S = P.solver()
+        assert S.planes == 4
+        o = S.block_order()
+        S.close()
+        assert len(o) == blocks
+        if blocks:
+            assert np.array_equal(np.sort(o), np.arange(blocks)) and np.array_equal(o[:bc_blocks], np.arange(bc_blocks))
+    finally:
+        P.close()
