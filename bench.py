@@ -125,7 +125,7 @@ def run_cpu_baseline_subprocess(steps=5000, warmup=5, reps=5, single_thread_step
 
 def dropin_call_us(P, n=50):
     """Wall time per call of the reference-surface entry points on the problem's device
-    arrays (each call ends with a device synchronize, as a C caller sees it)."""
+    arrays (each call returns when its work is done, as a C caller sees it)."""
     import ctypes as C
     from nrpyelliptic_amd import runtime
     L = runtime.lib()
@@ -528,7 +528,7 @@ def main():
                 "seconds": r_et.seconds, "log10_l2": r_et.log10_l2, "converged": bool(r_et.converged)}
     # per-launch kernel durations (back-to-back launches, HIP events on the solver stream): the
     # two-substep kernels of the production path, and the one-substep kernels with the RK4 step
-    # they make (the path of the Sommerfeld BC and of grids the two-substep kernel does not take)
+    # they make (the path of substeps_per_launch = 1)
     stage_us = {"stages12": round(S.time_substep(5, 200), 3), "stages34": round(S.time_substep(6, 200), 3)}
     S1 = P.solver(steps_per_graph=100, substeps_per_launch=1)
     stage_us.update({f"one_substep_stage{k}": round(S1.time_substep(k if k > 1 else 0, 200), 3) for k in (1, 2, 3, 4)})

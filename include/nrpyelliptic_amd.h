@@ -11,7 +11,9 @@
  *     by this library's MoL_malloc_* / rfm_precompute_rfmstruct_malloc;
  *   - xx[3] coordinate arrays and bc_struct tables stay in HOST memory, exactly as the
  *     reference lays them out (bcstruct_set_up output is byte-identical).
- * Every entry point is synchronous on return, like the reference's OpenMP functions.
+ * Every entry point is synchronous on return, like the reference's OpenMP functions: its own
+ * work and all earlier work of the default stream are done. Work of the caller's on other
+ * non-blocking streams is not waited for (nrpyell_device_synchronize waits for all).
  * Fatal errors print to stderr and exit(1), as the reference does
  * (bcstruct_set_up.c:178-184,272-277); HIP errors are reported the same way.
  *

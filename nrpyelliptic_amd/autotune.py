@@ -4,9 +4,10 @@ strength eta (EtaTuner) and, for an absolute accuracy bar, the damping schedule 
 Tile width of the fused RK4 substep kernel:
 
 The fused kernel puts i0 across the lanes of a 256-thread block (tile TX x 256/TX) and gives
-each thread one or two i2 planes; which shape keeps HBM busiest depends on N0 (ragged last
-tile, BC-tile share) and on the number of blocks per launch. This module times whole
-graph-replayed RK4 steps (the four fused launches with the residual check, as the solver runs
+each thread one or two i2 planes (or four, which the library chooses by itself where planes are
+left open and which has no number to ask for, so it is no candidate here); which shape keeps HBM
+busiest depends on N0 (ragged last tile, BC-tile share) and on the number of blocks per launch.
+This module times whole graph-replayed RK4 steps (with the residual check, as the solver runs
 them) for each candidate shape on the configuration's own grid, restoring the configuration's
 state afterwards, and caches the winner per (N0, N1, N2, precision) in a JSON file, so a batch
 of configurations is grouped by shape without re-timing shapes it has already seen. (Timing

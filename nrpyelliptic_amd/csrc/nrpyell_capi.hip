@@ -99,6 +99,8 @@ static T *halloc_mapped(size_t n, T **dev) {
 // one's stores are visible when it ends, so the flag says that all of the stream's earlier work is done.
 // At 128 x 128 x 16: L2_norm_of_gf 15.5 -> 13.1 us, MoL_step_forward_in_time 51 -> 36.3 us, a driver step of
 // three calls 86 -> 65 us.
+// The caller's other non-blocking streams are not waited for (hipDeviceSynchronize, which waits for them, takes
+// as long behind the flag as by itself: 18.2 us for the empty kernel).
 // A wait longer than SPIN_US, where this no longer matters and the CPU should not be held, goes on in
 // hipStreamSynchronize, which also reports a failed stream.
 static constexpr double SPIN_US = 150.0;
@@ -1158,8 +1160,8 @@ extern "C" void nrpyell_default_options(nrpyell_solve_options *o) {
 }
 
 // Four planes per thread (two-substep kernel, 32-wide tiles): the window of planes per thread is 14
-// for 4 points instead of 12 for 2, a quarter fewer vector loads, whose rate bounds the kernel once
-// many blocks hide its latencies (texture data unit 66 / 76 % busy at 256x256x32); but it takes 168 / 241
+// for 4 points instead of 12 for 2, a quarter fewer vector loads (the texture data unit is the busiest one
+// on large grids: 68 / 75 % of the stages-1+2 / 3+4 launch at 256x256x32); but it takes 168 / 241
 // registers, so two of its blocks fit a CU where three of the others do. For a grid alone it pays in
 // these ranges (four-plane blocks; BC blocks; us per RK4 step with two / four planes, FP64):
 // - 1.75 to 2 blocks per CU: with the BC blocks no more than three per CU (448; 224 128x224x16 33.9 / 30.8, 480; 192
@@ -1813,8 +1815,8 @@ extern "C" void MoL_step_forward_in_time(griddata_struct *griddata, const REAL d
 }
 
 // ---------------------------------------------------------------------------------------
-// Batched solver: many configurations (each its own grid shape) relaxed together, one
-// launch per RK4 substep per tile width, each configuration stopping on its own residual.
+// Batched solver: many configurations (each its own grid shape) relaxed together, one launch
+// per two RK4 substeps (or per one) and tile shape, each configuration stopping on its own residual.
 // ---------------------------------------------------------------------------------------
 __global__ void gather_state_kernel(SolverDeviceState *const *states, int n, double *out) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;

@@ -145,7 +145,7 @@ struct SubstepArgs {
   T eta, dt;
   const int *done;  // nonzero: converged, every launch returns at once
   int tx;           // tile width along i0 (threads), tile height along i1 = blockDim/tx
-  int pl;           // i2 planes per thread (1 or 2)
+  int pl;           // i2 planes per thread (1, 2 or 4; the one-substep kernel 1 or 2)
   int bc_rows;      // rows per BC block
   int nbc_rows;     // BC blocks per i2 plane: ceil(N1 / bc_rows)
   int ntile0, ntile1;

@@ -561,8 +561,9 @@ __global__ void mlp_adam_kernel(long n, const float *__restrict__ g, AdamArgs o)
 // bound by the activations' vector instructions (1280 per row, each an exponential, a reciprocal
 // and about 8 more; the MFMAs need 58 us of the 186 at 2.5 PFLOP/s) and overlaps them with other
 // waves' MFMAs: four blocks per CU, which the single buffer (40 KB of LDS) and 125 registers per
-// lane allow (one body for all five layers takes 160: layer 1 stands by itself). 262 144 rows: 186 us, 786 TFLOP/s (two ping-pong buffers, row-major weights loaded
-// where they are used and FP32 divisions: 390 us, 375 TFLOP/s; the same outputs).
+// lane allow (one body for all five layers takes 160: layer 1 stands by itself). 262 144 rows: 186 us,
+// 786 TFLOP/s (two ping-pong buffers, row-major weights loaded where they are used and FP32 divisions:
+// 390 us, 375 TFLOP/s; the same outputs).
 constexpr int FI_R = 64, FI_LD = MLP_W + 8;  // rows per block; LDS row stride (528 B)
 constexpr int FI_PF = 4;                     // inner steps of weights in flight
 

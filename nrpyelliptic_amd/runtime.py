@@ -545,8 +545,8 @@ class Solver:
 
 
 class BatchSolver:
-    """Relaxes many configurations (uneven grids) together on one GPU: one launch per RK4
-    substep per tile width covers the whole batch; each configuration stops at its own
+    """Relaxes many configurations (uneven grids) together on one GPU: one launch per two RK4
+    substeps and tile shape covers the whole batch; each configuration stops at its own
     residual target. `tiles` gives each configuration's tile as an i0 width or a
     (width, planes) pair (from the autotuner)."""
 
